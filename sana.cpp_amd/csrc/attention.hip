@@ -1644,15 +1644,22 @@ hipError_t linear_attention_chunked(const half_t * q, int64_t ldq, const half_t 
     return hipGetLastError();
 }
 
-size_t linattn_workspace_floats(int B, int N, int H, int D) {
-    const int T = la_chunk_tokens(N);
-    const size_t nch = (size_t)(N + T - 1) / T;
+namespace {
+size_t la_workspace_floats(int B, size_t nch, int H, int D) {
     const size_t E = (size_t)(D + 1) * D;
     const size_t NP = (size_t)(D + 1 + 31) / 32 * 32, KP = (size_t)(D + 15) / 16 * 16;
     // partial states (fp32, rounded up to 16 bytes) + the hi/lo fp16 state pair (counted in floats)
     // + the partials' maxima
     return ((size_t)B * H * E * nch + 3) / 4 * 4 + (size_t)B * H * NP * KP + (size_t)B * H * nch;
 }
+}  // namespace
+
+size_t linattn_workspace_floats(int B, int N, int H, int D) {
+    const int T = la_chunk_tokens(N);
+    return la_workspace_floats(B, (size_t)(N + T - 1) / T, H, D);
+}
+
+size_t linattn_workspace_floats_any(int B, int H, int D) { return la_workspace_floats(B, kLaChunks, H, D); }
 
 hipError_t linear_attention(const half_t * q, const half_t * k, const half_t * v, int64_t ld, half_t * out,
                             int64_t ldo, int B, int N, int H, int D, float * ws, hipStream_t s) {

@@ -431,8 +431,9 @@ void ensure_forward_buffers(sana_dit * c, int64_t B, int64_t N) {
         c->q16.ensure((size_t)M * C * 2);
         c->hid16.ensure((size_t)M * c->E * 2);
         c->glu16.ensure((size_t)M * c->Fp * 2);
-        c->la_ws.ensure(sana::linattn_workspace_floats((int)B, (int)N, (int)c->Hs, (int)c->Ds) * 4);
-        c->la_ws2.ensure(sana::linattn_workspace_floats(1, (int)N, (int)c->Hs, (int)c->Ds) * 4);
+        // for any token count: a later call of fewer tokens may split them into more chunks
+        c->la_ws.ensure(sana::linattn_workspace_floats_any((int)B, (int)c->Hs, (int)c->Ds) * 4);
+        c->la_ws2.ensure(sana::linattn_workspace_floats_any(1, (int)c->Hs, (int)c->Ds) * 4);
         c->d_t.ensure((size_t)B * 4);
         c->e1.ensure((size_t)B * C * 4);
         c->emb.ensure((size_t)B * C * 4);

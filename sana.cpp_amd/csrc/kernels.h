@@ -146,6 +146,9 @@ hipError_t final_layer(const float * x, const float * emb, const float * table, 
 // ReLU linear attention.  q/k/v fp16 token-major with row stride ld (head h at
 // columns h*D..), out fp16 with row stride ldo.  Workspace: partial states.
 size_t linattn_workspace_floats(int B, int N, int H, int D);
+// The same for every token count: the chunk count, and with it the size, is
+// not monotone in N (961 tokens make 16 chunks, 1089 make 9).
+size_t linattn_workspace_floats_any(int B, int H, int D);
 // Whole linear attention in one launch for head_dim 32, from the kGemmQKV
 // layouts: relu(q) token-major [B*N, ldq], relu(K)^T and V^T [B][H*32][N].
 bool linear_attention_fused_ok(int N, int D);

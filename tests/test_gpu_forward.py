@@ -360,3 +360,24 @@ def test_small_loop_graph_replays_match_direct_launches(small_model, monkeypatch
     assert np.array_equal(other, direct4)
     for r in replays:
         assert np.array_equal(r, direct6)
+
+
+def test_small_forward_fewer_tokens_more_chunks(small_model):
+    """31 x 31 tokens after 33 x 33: the linear attention splits the fewer
+    tokens into more chunks (16 against 9), so the workspace of the larger
+    forward must hold them; the result equals a fresh context's."""
+    import sana_dit
+    m, d = small_model
+    caption = O.randn((4, 16, 96), 31)
+    lat33, lat31 = O.randn((2, 8, 33, 33), 32), O.randn((2, 8, 31, 31), 33)
+    e = sana_dit.Dit(layers=2, hidden=128, ffn=256, caption_dim=96, latent_channels=8, self_heads=4, cross_heads=2)
+    try:
+        for name, shape in sana_dit.manifest(2, 128, 256, 96, 8).items():
+            e.set_weight(name, m.get(name, shape))
+        e.set_context(caption, projected=False)
+        ref = e.forward(lat31, 999.0)
+    finally:
+        e.close()
+    d.set_context(caption, projected=False)
+    d.forward(lat33, 999.0)
+    assert np.array_equal(d.forward(lat31, 999.0), ref)
