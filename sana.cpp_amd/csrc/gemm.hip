@@ -65,15 +65,20 @@ SANA_DEV void wait_vmcnt() {
 // s_waitcnt lgkmcnt(0): every LDS read of this wave has returned.
 SANA_DEV void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14)); }
 
-template <int BM, int BN, int WM, int WN, int STAGES>
+// KG: k-groups of WM x WN waves.  Group g sums the g-th of KG runs of
+// consecutive k-tiles through its own part of every stage, and the groups'
+// sums are added in group order before the epilogue.
+template <int BM, int BN, int WM, int WN, int STAGES, int KG = 1>
 struct Cfg {
-    static constexpr int NW = WM * WN;
+    static constexpr int GW = WM * WN;  // waves per k-group
+    static constexpr int NW = GW * KG;
     static constexpr int NT = 64 * NW;
     static constexpr int WTM = BM / WM, WTN = BN / WN;
     static constexpr int TM = WTM / 32, TN = WTN / 32;
     static constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128;
-    static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
-    static constexpr int A_LOADS = BM / 8 / NW, B_LOADS = BN / 8 / NW;  // wave instructions per stage
+    static constexpr int SUB_BYTES = A_BYTES + B_BYTES;  // one k-tile
+    static constexpr int STAGE_BYTES = KG * SUB_BYTES;
+    static constexpr int A_LOADS = BM / 8 / GW, B_LOADS = BN / 8 / GW;  // wave instructions per stage
     static constexpr int LOADS = A_LOADS + B_LOADS;
     static constexpr int CPAD = 4;                                      // fp32 epilogue row padding
     // The fp32 epilogue tile is staged in LDS: whole when it fits in the operand
@@ -83,7 +88,9 @@ struct Cfg {
         (BM * (BN + CPAD) * 4 <= (RING_BYTES > 80 * 1024 ? RING_BYTES : 80 * 1024)) ? BM : WTM;
     static constexpr int EPI_BYTES = EPI_ROWS * (BN + CPAD) * 4;
     static constexpr int LDS_BYTES = (RING_BYTES > EPI_BYTES) ? RING_BYTES : EPI_BYTES;
-    static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "tile rows must split into 8-row wave loads");
+    static constexpr int PART_BYTES = GW * TM * TN * 4096;  // one k-group's sums
+    static_assert((KG - 1) * PART_BYTES <= LDS_BYTES, "k-group partial sums");
+    static_assert(BM % (8 * GW) == 0 && BN % (8 * GW) == 0, "tile rows must split into 8-row wave loads");
     static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of 32x32");
     static_assert(LOADS * STAGES < 64, "vmcnt range");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS");
@@ -92,21 +99,21 @@ struct Cfg {
 // Wait until at most `keep` stages (0 <= keep < STAGES) of this wave's loads are outstanding.
 template <int LOADS, int STAGES>
 SANA_DEV void wait_stages(int keep) {
-    if constexpr (STAGES >= 4) {
-        if (keep >= 3) { wait_vmcnt<3 * LOADS>(); return; }
+    if constexpr (STAGES <= 1) {
+        wait_vmcnt<0>();
+    } else {
+        if (keep >= STAGES - 1) wait_vmcnt<(STAGES - 1) * LOADS>();
+        else wait_stages<LOADS, STAGES - 1>(keep);
     }
-    if constexpr (STAGES >= 3) {
-        if (keep >= 2) { wait_vmcnt<2 * LOADS>(); return; }
-    }
-    if (keep >= 1) { wait_vmcnt<LOADS>(); return; }
-    wait_vmcnt<0>();
 }
 
 // CONV: 0 plain A rows; 1 implicit 3x3 conv over a zero-bordered NHWC input;
 // 2 the same over the nearest-2x upsample of the input (GemmParams::conv).
-template <int BM, int BN, int WM, int WN, int STAGES, int MODE, int SCHED, int ACT, int CONV = 0>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
-    using G = Cfg<BM, BN, WM, WN, STAGES>;
+template <int BM, int BN, int WM, int WN, int STAGES, int MODE, int SCHED, int ACT, int CONV = 0, int KG = 1,
+          int SEG = 1>
+__global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in) {
+    using G = Cfg<BM, BN, WM, WN, STAGES, KG>;
+    static_assert((KG == 1 || SCHED == 1) && (SEG == 1 || (KG == 1 && SCHED != 0 && SCHED != 2)), "schedule");
     // product blockIdx.y of a batched launch (plain stores only)
     GemmParams p = p_in;
     if constexpr (MODE == kGemmStore && CONV == 0) {
@@ -136,7 +143,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wid = tid >> 6;
-    const int wm = wid / WN, wn = wid % WN;
+    const int kg = KG == 1 ? 0 : wid / G::GW, wi = KG == 1 ? wid : wid % G::GW;  // k-group, wave within it
+    const int wm = wi / WN, wn = wi % WN;
+    const int KT = p.K / kBK;
+    const int NT_K = (KT + KG - 1) / KG;  // k-tiles per group
 
     // Per-lane global source of each wave load (row clamped into range; the
     // rows past M / N are computed but never stored).
@@ -149,10 +159,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
     int cy[CONV ? G::A_LOADS : 1], cx[CONV ? G::A_LOADS : 1];
 #pragma unroll
     for (int i = 0; i < G::A_LOADS; ++i) {
-        const int r = (wid + i * G::NW) * 8 + lrow;
+        const int r = (wi + i * G::GW) * 8 + lrow;
         const int m = min(m0 + r, p.M - 1);
         if constexpr (CONV == 0) {
-            asrc[i] = reinterpret_cast<const f16 *>(p.A) + (int64_t)m * p.lda + lchunk(wid + i * G::NW) * 8;
+            asrc[i] = reinterpret_cast<const f16 *>(p.A) + (int64_t)m * p.lda + lchunk(wi + i * G::GW) * 8;
         } else {
             const int hw = p.conv_h * p.conv_w;
             const int img = m / hw, rem = m - img * hw;
@@ -160,22 +170,24 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
             cx[i] = rem - cy[i] * p.conv_w;
             const int ih = CONV == 2 ? p.conv_h / 2 : p.conv_h, iw = CONV == 2 ? p.conv_w / 2 : p.conv_w;
             asrc[i] = reinterpret_cast<const f16 *>(p.A) + (int64_t)img * (ih + 2) * (iw + 2) * p.lda +
-                      lchunk(wid + i * G::NW) * 8;
+                      lchunk(wi + i * G::GW) * 8;
         }
     }
 #pragma unroll
     for (int i = 0; i < G::B_LOADS; ++i) {
-        const int r = (wid + i * G::NW) * 8 + lrow;
-        bsrc[i] = reinterpret_cast<const f16 *>(p.W) + (int64_t)min(n0 + r, p.N - 1) * p.ldw + lchunk(wid + i * G::NW) * 8;
+        const int r = (wi + i * G::GW) * 8 + lrow;
+        bsrc[i] = reinterpret_cast<const f16 *>(p.W) + (int64_t)min(n0 + r, p.N - 1) * p.ldw + lchunk(wi + i * G::GW) * 8;
     }
     auto issue = [&](int kt, int st) {
-        unsigned char * base = smem + st * G::STAGE_BYTES;
+        unsigned char * base = smem + st * G::STAGE_BYTES + kg * G::SUB_BYTES;
+        // this group's k-tile (past the last one: the last again, never multiplied)
+        if constexpr (KG > 1) kt = min(kg * NT_K + kt, KT - 1);
         const int k0 = kt * kBK;
         if constexpr (CONV == 0) {
 #pragma unroll
             for (int i = 0; i < G::A_LOADS; ++i)
                 __builtin_amdgcn_global_load_lds(static_cast<const void *>(asrc[i] + k0),
-                                                 SANA_LDS(base + (wid + i * G::NW) * 1024), 16, 0, 0);
+                                                 SANA_LDS(base + (wi + i * G::GW) * 1024), 16, 0, 0);
         } else {
             // k-tile kt = (tap, 64-channel chunk): one 128-byte run of the source pixel
             const int cpt = (int)(p.lda >> 6);
@@ -197,12 +209,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
                     wp = p.conv_w / 2 + 2;
                 }
                 __builtin_amdgcn_global_load_lds(static_cast<const void *>(asrc[i] + ((int64_t)sr * wp + sc) * p.lda + c0),
-                                                 SANA_LDS(base + (wid + i * G::NW) * 1024), 16, 0, 0);
+                                                 SANA_LDS(base + (wi + i * G::GW) * 1024), 16, 0, 0);
             }
         }
 #pragma unroll
         for (int i = 0; i < G::B_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds(static_cast<const void *>(bsrc[i] + k0), SANA_LDS(base + G::A_BYTES + (wid + i * G::NW) * 1024),
+            __builtin_amdgcn_global_load_lds(static_cast<const void *>(bsrc[i] + k0), SANA_LDS(base + G::A_BYTES + (wi + i * G::GW) * 1024),
                                              16, 0, 0);
     };
 
@@ -227,7 +239,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
     constexpr int NB = (SCHED == 1 || SCHED == 3) ? NS : 2;    // fragment buffers
     f16x8 af[NB][G::TM], bf[NB][G::TN];
     auto load_frags = [&](int stage, int s, int buf) {
-        const unsigned char * sa = smem + stage * G::STAGE_BYTES;
+        const unsigned char * sa = smem + stage * G::STAGE_BYTES + kg * G::SUB_BYTES;
         const unsigned char * sb = sa + G::A_BYTES;
         const int ch = 2 * s + khalf;
 #pragma unroll
@@ -251,6 +263,32 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
         for (int i = 0; i < G::TM; ++i)
 #pragma unroll
             for (int j = 0; j < G::TN; ++j) acc[i][j] = mfma_32x32x16(bf[buf][j], af[buf][i], acc[i][j]);
+    };
+
+    // SEG > 1: the sums of SEG runs of consecutive k-tiles, added in run order --
+    // the order of SEG k-groups, so that kernels of either kind agree bit for bit.
+    f32x16 tot[SEG > 1 ? G::TM : 1][SEG > 1 ? G::TN : 1];
+    if constexpr (SEG > 1) {
+#pragma unroll
+        for (int i = 0; i < G::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < G::TN; ++j) tot[i][j] = acc[i][j];
+    }
+    int run_left = (KT + SEG - 1) / SEG;  // k-tiles of the current run still to come
+    auto fold = [&]() {
+        if constexpr (SEG > 1) {
+            if (--run_left) return;
+            run_left = (KT + SEG - 1) / SEG;
+#pragma unroll
+            for (int i = 0; i < G::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < G::TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        tot[i][j][r] += acc[i][j][r];
+                        acc[i][j][r] = 0.0f;
+                    }
+        }
     };
 
     // Residual epilogue inputs (x rows and the gate), loaded before the main loop
@@ -331,11 +369,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
         }
     }
 
-    const int KT = p.K / kBK;
 #pragma unroll
     for (int s = 0; s < STAGES; ++s)
-        if (s < KT) issue(s, s);
-    wait_stages<G::LOADS, STAGES>(min(STAGES - 1, KT - 1));
+        if (s < NT_K) issue(s, s);
+    wait_stages<G::LOADS, STAGES>(min(STAGES - 1, NT_K - 1));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (SCHED == 3) {
@@ -344,11 +381,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
         // refilled with tile kt+STAGES before the tile's MFMAs run.  With two
         // stages, two tiles of DMA are in flight during the MFMAs instead of one,
         // which hides the longer latency of weights that come from HBM.
-        for (int kt = 0; kt < KT; ++kt) {
+        for (int kt = 0; kt < NT_K; ++kt) {
             const int st = kt % STAGES;
             if (kt > 0) {
                 __builtin_amdgcn_sched_barrier(0);
-                wait_stages<G::LOADS, STAGES>(min(STAGES - 1, KT - 1 - kt));
+                wait_stages<G::LOADS, STAGES>(min(STAGES - 1, NT_K - 1 - kt));
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -358,26 +395,30 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
             wait_lgkmcnt0();
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
-            if (kt + STAGES < KT) issue(kt + STAGES, st);
+            if (kt + STAGES < NT_K) issue(kt + STAGES, st);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < NS; ++s) mfmas(s);
+            fold();
         }
     } else if constexpr (SCHED == 1) {
         // every fragment of the tile is requested right after the barrier; the
         // MFMAs of step s wait only for the reads of steps <= s (in-order lgkmcnt)
-        for (int kt = 0; kt < KT; ++kt) {
+        for (int kt = 0; kt < NT_K; ++kt) {
             const int st = kt % STAGES;
+            if (KG == 1 || kg * NT_K + kt < KT) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) load_frags(st, s, s);
+                for (int s = 0; s < NS; ++s) load_frags(st, s, s);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) mfmas(s);
-            if (kt + 1 < KT) {
+                for (int s = 0; s < NS; ++s) mfmas(s);
+            }
+            fold();
+            if (kt + 1 < NT_K) {
                 __builtin_amdgcn_sched_barrier(0);
-                wait_stages<G::LOADS, STAGES>(min(STAGES - 2, KT - 2 - kt));
+                wait_stages<G::LOADS, STAGES>(min(STAGES - 2, NT_K - 2 - kt));
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_sched_barrier(0);
-                if (kt + STAGES < KT) issue(kt + STAGES, st);
+                if (kt + STAGES < NT_K) issue(kt + STAGES, st);
             }
         }
     } else {
@@ -386,7 +427,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
         // boundary (wait for the next tile's DMA, barrier, refill the freed
         // stage) follows the last step's MFMAs, so it overlaps them.
         load_frags(0, 0, 0);
-        for (int kt = 0; kt < KT; ++kt) {
+        for (int kt = 0; kt < NT_K; ++kt) {
             const int st = kt % STAGES;
 #pragma unroll
             for (int s = 0; s < NS - 1; ++s) {
@@ -398,16 +439,57 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
                 }
             }
             mfmas((NS - 1) & 1);
-            if (kt + 1 < KT) {
+            if (kt + 1 < NT_K) {
                 __builtin_amdgcn_sched_barrier(0);
                 // tile kt+1 has landed (this wave's DMA), then every wave's has and
                 // every wave is done reading stage st, which takes tile kt+STAGES.
-                wait_stages<G::LOADS, STAGES>(min(STAGES - 2, KT - 2 - kt));
+                wait_stages<G::LOADS, STAGES>(min(STAGES - 2, NT_K - 2 - kt));
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_sched_barrier(0);
-                if (kt + STAGES < KT) issue(kt + STAGES, st);
+                if (kt + STAGES < NT_K) issue(kt + STAGES, st);
                 load_frags((kt + 1) % STAGES, 0, 0);
             }
+        }
+    }
+
+    if constexpr (SEG > 1) {  // the last run (all zeros where it was folded above)
+#pragma unroll
+        for (int i = 0; i < G::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < G::TN; ++j) acc[i][j] += tot[i][j];
+    }
+    // groups 1.. hand their sums to group 0 through LDS, lane by lane; group 0
+    // adds them in group order and runs the epilogue's staging
+    if constexpr (KG > 1) {
+        float4 * part = reinterpret_cast<float4 *>(smem);
+        constexpr int PF4 = G::PART_BYTES / 16;
+        __syncthreads();  // every wave is done reading the operand ring
+        if (kg > 0) {
+#pragma unroll
+            for (int i = 0; i < G::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < G::TN; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        part[(kg - 1) * PF4 + ((wi * G::TM + i) * G::TN + j) * 256 + q * 64 + lane] = make_float4(
+                            acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        }
+        __syncthreads();
+        if (kg == 0) {
+#pragma unroll
+            for (int i = 0; i < G::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < G::TN; ++j)
+#pragma unroll
+                    for (int h = 0; h < KG - 1; ++h)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const float4 v = part[h * PF4 + ((wi * G::TM + i) * G::TN + j) * 256 + q * 64 + lane];
+                            acc[i][j][4 * q] += v.x;
+                            acc[i][j][4 * q + 1] += v.y;
+                            acc[i][j][4 * q + 2] += v.z;
+                            acc[i][j][4 * q + 3] += v.w;
+                        }
         }
     }
 
@@ -438,6 +520,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
             static_assert(BM * LDH * 2 <= G::LDS_BYTES, "fp16 epilogue tile");
             f16 * ht = reinterpret_cast<f16 *>(smem);
             __syncthreads();  // every wave is done reading the operand ring
+            if (KG == 1 || kg == 0) {  // the k-group that holds the sums
 #pragma unroll
             for (int j = 0; j < G::TN; ++j)
 #pragma unroll
@@ -465,6 +548,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
                         *reinterpret_cast<f16x4 *>(ht + row * LDH + c) = h;
                     }
                 }
+            }
             __syncthreads();
             // row-major stores (the whole tile, or the q section of the split)
             constexpr int HCPR = BN / 8, CHUNKS = BM * HCPR;
@@ -556,7 +640,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmParams p_in) {
         }
         for (int pass = 0; pass < BM / ER; ++pass) {
             __syncthreads();  // the operand ring (pass 0) or the previous pass's rows are free
-            if (ER == BM || wm == pass) {
+            if ((KG == 1 || kg == 0) && (ER == BM || wm == pass)) {
                 // 16-byte row runs (rows are 16-byte aligned: LDC = BN + 4, BN a multiple of 8)
 #pragma unroll
                 for (int i = 0; i < G::TM; ++i)
@@ -813,18 +897,20 @@ bool set_lds_limit(const void * k, size_t lds) {
     return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, int MODE, int SCHED, int ACT, int CONV = 0>
+template <int BM, int BN, int WM, int WN, int STAGES, int MODE, int SCHED, int ACT, int CONV = 0, int KG = 1,
+          int SEG = 1>
 hipError_t launch_mode(const GemmParams & p, int tiles, hipStream_t s) {
-    using G = Cfg<BM, BN, WM, WN, STAGES>;
+    using G = Cfg<BM, BN, WM, WN, STAGES, KG>;
     static const bool attr = set_lds_limit(
-        reinterpret_cast<const void *>(&gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV>), G::LDS_BYTES);
+        reinterpret_cast<const void *>(&gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV, KG, SEG>), G::LDS_BYTES);
     (void)attr;
     static const std::string name = "gemm_kernel<" + std::to_string(BM) + ", " + std::to_string(BN) + ", " +
                                     std::to_string(WM) + ", " + std::to_string(WN) + ", " + std::to_string(STAGES) +
                                     ", " + std::to_string(MODE) + ", " + std::to_string(SCHED) + ", " +
-                                    std::to_string(ACT) + ", " + std::to_string(CONV) + ">";
+                                    std::to_string(ACT) + ", " + std::to_string(CONV) + ", " +
+                                    std::to_string(KG) + ", " + std::to_string(SEG) + ">";
     note_kernel(name.c_str());
-    hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV>), dim3(tiles, p.batch), dim3(G::NT),
+    hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV, KG, SEG>), dim3(tiles, p.batch), dim3(G::NT),
                        G::LDS_BYTES, s, p);
     return hipGetLastError();
 }
@@ -843,6 +929,35 @@ template <int BM, int BN, int WM, int WN, int STAGES, int SCHED>
 hipError_t launch_conv(const GemmParams & p, hipStream_t s) {
     if (p.conv == 2) return launch_conv_mode<BM, BN, WM, WN, STAGES, SCHED, 2>(p, s);
     return launch_conv_mode<BM, BN, WM, WN, STAGES, SCHED, 1>(p, s);
+}
+
+// Few-tile grids: k-groups (stores, residual updates, the q|k|v split).
+template <int BM, int BN, int WM, int WN, int STAGES, int KG>
+hipError_t launch_kg(const GemmParams & p, hipStream_t s) {
+    const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+    if (p.mode == kGemmResidual)
+        return launch_mode<BM, BN, WM, WN, STAGES, kGemmResidual, 1, kActNone, 0, KG>(p, tiles, s);
+    if (p.mode == kGemmQKV) return launch_mode<BM, BN, WM, WN, STAGES, kGemmQKV, 1, kActNone, 0, KG>(p, tiles, s);
+    if (p.act == kActSilu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActSilu, 0, KG>(p, tiles, s);
+    if (p.act == kActGelu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActGelu, 0, KG>(p, tiles, s);
+    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActNone, 0, KG>(p, tiles, s);
+}
+
+// Plain stores whose k sums are four runs added in order (GemmParams::k_runs):
+// four k-groups, or one group that folds its sums.
+template <int BM, int BN, int WM, int WN, int STAGES, int SCHED, int KG>
+hipError_t launch_runs(const GemmParams & p, hipStream_t s) {
+    const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, SCHED, kActNone, 0, KG, 4 / KG>(p, tiles, s);
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES, int CONV, int KG>
+hipError_t launch_conv_kg(const GemmParams & p, hipStream_t s) {
+    const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+    if (p.mode == kGemmResidual)
+        return launch_mode<BM, BN, WM, WN, STAGES, kGemmResidual, 1, kActNone, CONV, KG>(p, tiles, s);
+    if (p.act == kActSilu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActSilu, CONV, KG>(p, tiles, s);
+    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActNone, CONV, KG>(p, tiles, s);
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int SCHED = 0>
@@ -894,6 +1009,8 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
          ((reinterpret_cast<uintptr_t>(p.kt16) | reinterpret_cast<uintptr_t>(p.vt16)) & 15)))
         return hipErrorInvalidValue;
     if (p.gate_a && p.rows_per_batch <= 0) return hipErrorInvalidValue;
+    if (p.k_runs != 1 && (p.k_runs != 4 || p.mode != kGemmStore || p.conv || p.act != kActNone))
+        return hipErrorInvalidValue;
     if (p.batch < 1 || p.batch > 65535 || p.batch_w_div < 1 ||
         (p.batch > 1 && (p.mode != kGemmStore || p.conv ||
                          ((p.batch_a | p.batch_w | p.batch_o16 | p.batch_o32) & 7) != 0)))
@@ -906,7 +1023,15 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     if (p.gate_t) vec = vec && (reinterpret_cast<uintptr_t>(p.gate_t) & 15) == 0;
     if (p.bias) vec = vec && (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0;
     p.vec = vec ? 1 : 0;
+    const int64_t co = std::max(p.co, 1) * (int64_t)p.batch;
+    // tiles of the rows that decide the order of the k sums
+    const int64_t rows = p.order_rows > 0 ? p.order_rows : p.M;
+    auto grid = [&](int bm, int bn) { return (rows + bm - 1) / bm * ((p.N + bn - 1) / bn) * co; };
     if (p.conv) {
+        if (grid(32, 64) <= 288)
+            return p.conv == 2 ? launch_conv_kg<32, 64, 1, 2, 3, 2, 4>(p, s) : launch_conv_kg<32, 64, 1, 2, 3, 1, 4>(p, s);
+        if (grid(64, 64) <= 320)
+            return p.conv == 2 ? launch_conv_kg<64, 64, 2, 2, 4, 2, 2>(p, s) : launch_conv_kg<64, 64, 2, 2, 4, 1, 2>(p, s);
         // Early stage release is 2-6 % faster than schedule 1 on the VAE's
         // 3x3 convs (1024^2 x 128, 512^2 x 256, 256^2 x 512) but 15 % slower
         // on the upsampling convs, whose residual epilogue reads the shortcut.
@@ -942,7 +1067,34 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     //  16384 rows per branch 54.00 -> 53.66 ms, at 1024 rows 5.089 -> 5.081 ms.
     // (tile counts are scaled by the launches that share the CUs, p.co, and
     // by the products of a batched launch)
-    const int64_t co = std::max(p.co, 1) * (int64_t)p.batch;
+    // Grids of few tiles leave most CUs idle and each workgroup with a chain of
+    // K / 64 tile latencies (0.44 us each); k-groups cut the chain and keep more
+    // bytes in flight per CU.  The smallest tiles that still fit about one
+    // workgroup per CU; graph chains, us per launch, before -> after (M x N x K):
+    //  128 x 1152 x 1152 residual 11.5 -> 6.4, K = 2880 18.3 -> 9.6 (32x32, 4 groups);
+    //  143 x 3072 x 1024 9.8 -> 6.3 (32x64, 4 groups); 512 x 1152 x 1152 store
+    //  10.7 -> 7.8, residual K = 2880 19.1 -> 15.3 (64x64, 2 groups).  From 1.3
+    //  workgroups per CU on (324 64x64 tiles) the gain is 3 % and falls to none.
+    //  Sums that may not depend on M (the text encoder) take k_runs: 23 x 4096 x
+    //  2304 15.2 -> 9.3, 23 x 2304 x 2304 15.2 -> 8.7; folding the same four runs
+    //  in one group costs 738-row launches 0-2 %.  Its gate | up product keeps k
+    //  in one sequence; up to 32 rows one-wave 32x32 tiles stream its weights at
+    //  4.5 TB/s (27.0 -> 19.1 us).
+    if (p.k_runs == 4) {
+        if (grid(32, 32) <= 256) return launch_runs<32, 32, 1, 1, 3, 1, 4>(p, s);
+        if (p.M > 32 && p.M <= 64 && grid(64, 32) <= 256) return launch_runs<64, 32, 2, 1, 3, 1, 4>(p, s);
+        if (grid(32, 64) <= 256) return launch_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
+        if (grid(64, 64) <= 256) return launch_runs<64, 64, 2, 2, 2, 1, 4>(p, s);
+        if (grid(128, 128) > 256) return launch_runs<128, 128, 4, 2, 2, 1, 1>(p, s);
+        if (grid(128, 64) >= 256) return launch_runs<128, 64, 2, 2, 2, 3, 1>(p, s);
+        return launch_runs<64, 64, 2, 2, 3, 1, 1>(p, s);
+    }
+    if (p.order_rows >= 0 && p.K >= 512 && p.batch == 1 && p.mode != kGemmVT && p.act != kActGeglu) {
+        if (grid(32, 32) <= 256) return launch_kg<32, 32, 1, 1, 3, 4>(p, s);
+        if (grid(32, 64) <= 288) return launch_kg<32, 64, 1, 2, 3, 4>(p, s);
+        if (grid(64, 64) <= 256) return launch_kg<64, 64, 2, 2, 4, 2>(p, s);
+    }
+    if (p.M <= 32 && p.mode == kGemmStore && p.N >= 8192) return launch<32, 32, 1, 1, 4, 1>(p, s);
     const int64_t tm128 = (p.M + 127) / 128;
     const int64_t t128 = tm128 * ((p.N + 127) / 128) * co;
     if (t128 <= 160) {
@@ -954,13 +1106,12 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     }
     if (t128 <= 256 && tm128 * ((p.N + 63) / 64) * co >= 256) return launch<128, 64, 2, 2, 2, 3>(p, s);
     const int64_t tn128 = (p.N + 127) / 128;
-    if (co == 1 && std::min(tm128, tn128) <= 5 && std::max(tm128, tn128) >= 128)
-        return launch<128, 128, 4, 2, 2, 1>(p, s);
     const int64_t t192 = p.N % 192 == 0 ? tm128 * (p.N / 192) * co : 0;
     constexpr int64_t kSlots = 512;
-    if (t192 >= kSlots * 3 / 2 ||
-        (p.mode == kGemmStore && p.N >= 3456 && t192 > 0 && t192 <= kSlots && t128 > kSlots))
-    {
+    const bool one_round192 = p.mode == kGemmStore && p.N >= 3456 && t192 > 0 && t192 <= kSlots && t128 > kSlots;
+    if (!one_round192 && co == 1 && std::min(tm128, tn128) <= 5 && std::max(tm128, tn128) >= 128)
+        return launch<128, 128, 4, 2, 2, 1>(p, s);
+    if (t192 >= kSlots * 3 / 2 || one_round192) {
         if (p.mode == kGemmQKV || (p.mode == kGemmResidual && p.K <= 1152)) return launch<128, 192, 4, 2, 2, 1>(p, s);
         return launch<128, 192, 2, 2, 2, 1>(p, s);
     }

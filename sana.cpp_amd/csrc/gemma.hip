@@ -407,9 +407,13 @@ void ensure_workspace(sana_gemma * g, const std::vector<Seq> & q) {
 }
 
 void gemm(const half_t * A, int64_t lda, const half_t * W, int64_t ldw, int64_t M, int64_t N, int64_t K,
-          half_t * o16, int64_t ldo16, float * o32, int64_t ldo32, hipStream_t s, int act = sana::kActNone) {
+          half_t * o16, int64_t ldo16, float * o32, int64_t ldo32, hipStream_t s, int act = sana::kActNone,
+          int runs = 1) {
     sana::GemmParams p;
     p.act = act;
+    // a row's sums must not depend on the rows encoded with it
+    p.order_rows = -1;
+    p.k_runs = runs;
     p.A = A;
     p.lda = lda;
     p.W = W;
@@ -428,8 +432,10 @@ void gemm(const half_t * A, int64_t lda, const half_t * W, int64_t ldw, int64_t 
 // writes o16 + z * so16 / o32 + z * so32.
 void gemm_batched(const half_t * A, int64_t lda, int64_t sa, const half_t * W, int64_t ldw, int64_t sw, int wdiv,
                   int64_t M, int64_t N, int64_t K, half_t * o16, int64_t ldo16, int64_t so16, float * o32,
-                  int64_t ldo32, int64_t so32, int batch, hipStream_t s) {
+                  int64_t ldo32, int64_t so32, int batch, hipStream_t s, int runs = 1) {
     sana::GemmParams p;
+    p.order_rows = -1;
+    p.k_runs = runs;
     p.A = A;
     p.lda = lda;
     p.W = W;
@@ -481,6 +487,11 @@ int split_k(int64_t K) {
     return K % 128 == 0 && K / 2 >= 512 ? 2 : 1;
 }
 
+// Runs of k-tiles that a long contraction is summed in (GemmParams::k_runs):
+// few-row encodes sum them side by side, where k in one sequence is a chain of
+// K / 64 tile latencies.  Depends on K only, as split_k.
+int k_runs(int64_t K) { return K >= 1024 ? 4 : 1; }
+
 // decode_embeddings (src/gemma_encoder.cpp:95-152) on device token ids, for
 // one or more independent sequences at once: their rows share every
 // per-token kernel (norms, the projections, GeGLU) and only the attention
@@ -501,7 +512,8 @@ void encode(sana_gemma * g, const std::vector<Seq> & seqs, hipStream_t s) {
         // the pre-attention norm: layer 0 here, later layers in the previous
         // layer's last norm launch
         if (l == 0) norm(g, g->x32.as<float>(), M, L.n_attn, 0, a16, nullptr, s);
-        gemm(a16, H, L.wqkv.as<half_t>(), H, M, Dqkv, H, nullptr, 0, g->qkv32.as<float>(), Dqkv, s);
+        gemm(a16, H, L.wqkv.as<half_t>(), H, M, Dqkv, H, nullptr, 0, g->qkv32.as<float>(), Dqkv, s, sana::kActNone,
+             k_runs(H));
         const int window = (c.sliding_window > 0 && l % 2 == 0) ? (int)c.sliding_window : 0;
         // sequences 1, 3, ... on the second stream (their buffers are disjoint)
         const bool two = seqs.size() > 1;
@@ -550,13 +562,13 @@ void encode(sana_gemma * g, const std::vector<Seq> & seqs, hipStream_t s) {
         }
         const int so = split_k(Dq);
         gemm_batched(g->o16.as<half_t>(), Dq, Dq / so, L.wo.as<half_t>(), Dq, Dq / so, 1, M, H, Dq / so, nullptr, 0,
-                     0, g->y32.as<float>(), H, M * H, so, s);
+                     0, g->y32.as<float>(), H, M * H, so, s, k_runs(Dq / so));
         // x += post-attention norm of the projection, then the pre-FFN norm
         norm(g, g->y32.as<float>(), M, L.n_post_attn, 3, a16, g->x32.as<float>(), s, so, &L.n_ffn);
         gemm(a16, H, L.wgu.as<half_t>(), H, M, 2 * F, H, g->g16.as<half_t>(), F, nullptr, 0, s, sana::kActGeglu);
         const int sd = split_k(F);
         gemm_batched(g->g16.as<half_t>(), F, F / sd, L.wdown.as<half_t>(), F, F / sd, 1, M, H, F / sd, nullptr, 0, 0,
-                     g->y32.as<float>(), H, M * H, sd, s);
+                     g->y32.as<float>(), H, M * H, sd, s, k_runs(F / sd));
         // x += post-FFN norm, then the next layer's pre-attention norm
         if (l + 1 < c.layers)
             norm(g, g->y32.as<float>(), M, L.n_post_ffw, 3, a16, g->x32.as<float>(), s, sd,

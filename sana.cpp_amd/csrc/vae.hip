@@ -476,8 +476,9 @@ std::vector<std::string> required_names(const sana_vae * v) {
 // decode
 
 void gemm_plain(const half_t * A, int64_t lda, const DevMem & W, int64_t M, int64_t N, int64_t K, const float * bias,
-                int act, half_t * out16, int64_t ldo16, float * out32, int64_t ldo32, hipStream_t s) {
+                int act, half_t * out16, int64_t ldo16, float * out32, int64_t ldo32, hipStream_t s, int64_t B) {
     sana::GemmParams p;
+    p.order_rows = (int)(M / B);  // a batch sums as its images alone do
     p.A = A;
     p.lda = lda;
     p.W = W.as<half_t>();
@@ -500,6 +501,7 @@ void gemm_conv(int conv, const half_t * A, int64_t cin, const DevMem & W, int64_
                int64_t N, const float * bias, int act, bool residual, float * x32, half_t * out16, bool pad16,
                float * out32, hipStream_t s, const float * up_src = nullptr, int64_t up_c = 0) {
     sana::GemmParams p;
+    p.order_rows = (int)(H * Wd);
     p.conv = conv;
     p.conv_h = (int)H;
     p.conv_w = (int)Wd;
@@ -662,7 +664,7 @@ void decode(sana_vae * v, const float * lat, int64_t B, int64_t h, int64_t w, fl
                 const int64_t heads = C / kVaeHead;
                 half_t * qkv = v->qkv16.as<half_t>();
                 gemm_plain(v->a16.as<half_t>(), C, a.wqkv, P, 3 * C, C, nullptr, sana::kActNone, qkv, 3 * C, nullptr,
-                           0, s);
+                           0, s, B);
                 {
                     const int64_t n = P * (3 * C / 8);
                     hipLaunchKernelGGL(vae_dw5x5_kernel, dim3(blocks_for(n)), dim3(256), 0, s,
@@ -683,17 +685,17 @@ void decode(sana_vae * v, const float * lat, int64_t B, int64_t h, int64_t w, fl
                                                     (int)(H * W), (int)heads, kVaeHead, v->la_ws.as<float>(), s),
                              "vae linear attention");
                 gemm_plain(mrg, 2 * C, a.wout, P, C, 2 * C, nullptr, sana::kActNone, nullptr, 0, v->t32.as<float>(), C,
-                           s);
+                           s, B);
                 rmsnorm(v->t32.as<float>(), C, P, a.anw, &a.anb, x, false, x, v->a16.as<half_t>(), false, H, W, s);
                 // GLUMBConv: inverted 1x1 (+ bias, SiLU), depthwise 3x3 + GLU, point 1x1
                 const int64_t Hd = v->expand * C;
                 gemm_plain(v->a16.as<half_t>(), C, a.winv, P, 2 * Hd, C, a.binv.as<float>(), sana::kActSilu,
-                           v->hid16.as<half_t>(), 2 * Hd, nullptr, 0, s);
+                           v->hid16.as<half_t>(), 2 * Hd, nullptr, 0, s, B);
                 launch_check(sana::dwconv_glu(v->hid16.as<half_t>(), 2 * Hd, a.wdw.as<float>(), a.bdw.as<float>(),
                                               v->glu16.as<half_t>(), Hd, (int)B, (int)H, (int)W, (int)Hd, s),
                              "vae dwconv glu");
                 gemm_plain(v->glu16.as<half_t>(), Hd, a.wpt, P, C, Hd, nullptr, sana::kActNone, nullptr, 0,
-                           v->t32.as<float>(), C, s);
+                           v->t32.as<float>(), C, s, B);
                 const bool to_pad = last && next_up;
                 rmsnorm(v->t32.as<float>(), C, P, a.gnw, &a.gnb, x, false, x,
                         to_pad ? cur->as<half_t>() : v->a16.as<half_t>(), to_pad, H, W, s);

@@ -62,6 +62,41 @@ GEMM_SHAPES = [
 ]
 
 
+# few-tile grids: k-groups of 32x32, 32x64 and 64x64 tiles; K / 64 a multiple of the groups or not
+KGROUP_SHAPES = [(1, 1152, 1152), (23, 1152, 2880), (33, 3456, 1152), (64, 1152, 2880), (65, 5760, 576),
+                 (256, 1152, 2880), (250, 1152, 1152), (529, 512, 704), (31, 70, 512), (144, 300, 640),
+                 (20, 8200, 2304)]
+
+
+@pytest.mark.parametrize("M,N,K", KGROUP_SHAPES)
+def test_gemm_k_groups(L, M, N, K):
+    """Stores (fp16 and fp32 out) and gated residual updates against fp64.  fp32
+    sums of K products: |error| <= (K + 8) 2^-24 sum |a w| in any order."""
+    rng = np.random.default_rng(M + N + K)
+    A, W = f16(rng.standard_normal((M, K))), f16(rng.standard_normal((N, K)) * 0.05)
+    bias = rng.standard_normal(N).astype(np.float32)
+    gate = rng.standard_normal((1, N)).astype(np.float32)
+    x = rng.standard_normal((M, N)).astype(np.float32)
+    ref = A.astype(np.float64) @ W.astype(np.float64).T + bias
+    mag = np.abs(A).astype(np.float64) @ np.abs(W).astype(np.float64).T + np.abs(bias)
+    dA, dW, db = dev(A, torch.float16), dev(W, torch.float16), dev(bias, torch.float32)
+    o32 = torch.empty((M, N), device="cuda", dtype=torch.float32)
+    o16 = torch.empty((M, N), device="cuda", dtype=torch.float16)
+    args = (dA.data_ptr(), K, dW.data_ptr(), K, M, N, K, db.data_ptr())
+    L.check(L.lib().sana_hip_gemm(*args, 0, o16.data_ptr(), N, o32.data_ptr(), N, stream()))
+    bound = (K + 8) * 2.0 ** -24 * mag
+    assert (np.abs(host(o32) - ref) <= bound).all()
+    L.check(L.lib().sana_hip_gemm(*args, 0, o16.data_ptr(), N, None, 0, stream()))
+    assert (np.abs(host(o16) - ref) <= bound + 2.0 ** -11 * np.abs(ref) + 2.0 ** -24).all()
+    dx, dg = dev(x, torch.float32), dev(gate, torch.float32)
+    L.check(L.lib().sana_hip_gemm_residual(*args, dg.data_ptr(), None, N, M, dx.data_ptr(), N, o16.data_ptr(), N,
+                                           stream()))
+    rx = x + gate.astype(np.float64) * ref
+    tol = np.abs(gate) * bound + 4 * 2.0 ** -24 * (np.abs(x) + np.abs(gate * ref))
+    assert (np.abs(host(dx) - rx) <= tol).all()
+    assert (np.abs(host(o16) - rx) <= tol + 2.0 ** -11 * np.abs(rx) + 2.0 ** -24).all()
+
+
 @pytest.mark.parametrize("M,N,K", GEMM_SHAPES)
 def test_gemm_store(L, M, N, K):
     rng = np.random.default_rng(M * 7 + N)
