@@ -21,6 +21,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -30,7 +31,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <tuple>
 #include <vector>
 
 #include "../../include/sana_dit.h"
@@ -77,10 +77,6 @@ __global__ void cfg_dpm_kernel(const float * __restrict__ np, const float * __re
     x0_out[i] = x0;
 }
 
-struct GraphEntry {
-    hipGraphExec_t exec = nullptr;
-};
-
 }  // namespace
 
 namespace sana {
@@ -97,7 +93,7 @@ struct sana_dit {
     int64_t C = 0, E = 0, F = 0, Ccap = 0, Cl = 0, L_ = 0, Hs = 0, Hc = 0, Ds = 0, Dc = 0;
     int64_t Cp = 0, Fp = 0, Ccap_p = 0;  // K-padded row strides of GEMM operands
     hipStream_t stream = nullptr;
-    // second branch of a CFG-split forward (the conditional batch row) and
+    // second chain of a forward (the second half of the CFG batch) and
     // its fork / join events; same (default) priority as `stream`
     hipStream_t stream2 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -121,24 +117,18 @@ struct sana_dit {
     DevMem x32, fin32, xa16, qkv16, o16, r16, q16, hid16, glu16, la_ws, la_ws2, d_t, e1, emb, tmod, mod_all,
         lat_in, np_out;
     DevMem loop_lat[2], loop_x0[2];  // denoise loop: latent ping-pong and converted-output history
-    // graphs keyed by (kind, Bl, H, W, L, pointers)
-    std::map<std::tuple<int, int64_t, int64_t, int64_t, int64_t, const void *, const void *, const void *, const void *>,
-             GraphEntry>
-        graphs;
-    // whole denoise loops, keyed by shape, buffers and schedule (a few kept)
-    std::map<std::string, GraphEntry> loop_graphs;
+    // block chains as graphs, keyed by (chain, chains, batch rows, tokens, keys, masked);
+    // they touch the context's own buffers only, so they are dropped where one is reallocated
+    std::map<std::array<int64_t, 6>, hipGraphExec_t> graphs;
     int64_t last_M = 0, last_B = 0, last_N = 0;
     int64_t loop_steps = 0, loop_n = 0;  // shape of the last denoise loop (its converted outputs stay in loop_x0)
     // Execution switches, read from the environment once by sana_dit_create:
-    // SANA_DIT_CFG_BRANCHES=0 runs the CFG pair as one chain, SANA_DIT_NO_GRAPH=1
-    // launches the forward's kernels directly instead of replaying a graph.
+    // SANA_DIT_CFG_BRANCHES=0 runs the CFG batch as one chain, SANA_DIT_NO_GRAPH=1
+    // launches the blocks' kernels directly instead of replaying graphs.
     bool cfg_branches = true, use_graphs = true;
 
     ~sana_dit() {
-        for (auto & kv : graphs)
-            if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
-        for (auto & kv : loop_graphs)
-            if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
+        for (auto & kv : graphs) (void)hipGraphExecDestroy(kv.second);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
         if (ev_head_fork) (void)hipEventDestroy(ev_head_fork);
@@ -152,17 +142,9 @@ struct sana_dit {
 
 namespace {
 
-void drop_loop_graphs(sana_dit * c) {
-    for (auto & kv : c->loop_graphs)
-        if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
-    c->loop_graphs.clear();
-}
-
 void drop_graphs(sana_dit * c) {
-    for (auto & kv : c->graphs)
-        if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
+    for (auto & kv : c->graphs) (void)hipGraphExecDestroy(kv.second);
     c->graphs.clear();
-    drop_loop_graphs(c);
 }
 
 // A weight upload: the captured graphs go, and so does the conditioning when
@@ -433,7 +415,7 @@ void ensure_forward_buffers(sana_dit * c, int64_t B, int64_t N) {
         c->glu16.ensure((size_t)M * c->Fp * 2);
         // for any token count: a later call of fewer tokens may split them into more chunks
         c->la_ws.ensure(sana::linattn_workspace_floats_any((int)B, (int)c->Hs, (int)c->Ds) * 4);
-        c->la_ws2.ensure(sana::linattn_workspace_floats_any(1, (int)c->Hs, (int)c->Ds) * 4);
+        c->la_ws2.ensure(sana::linattn_workspace_floats_any((int)((B + 1) / 2), (int)c->Hs, (int)c->Ds) * 4);
         c->d_t.ensure((size_t)B * 4);
         c->e1.ensure((size_t)B * C * 4);
         c->emb.ensure((size_t)B * C * 4);
@@ -501,12 +483,12 @@ void enqueue_block(sana_dit * c, int64_t i, int64_t B, int64_t N, const float * 
     // exceeds the 256 MB last-level cache), and a GEMM waits on its first
     // k-tiles the longer for it.  The two LN launches carry extra workgroups
     // that pull weights into that cache ahead of use: LN1 this block's cross
-    // and point weights, LN2 the next block's q|k|v and out weights.  CFG
-    // branches each read their share.  The inverted-FFN weights are left cold:
+    // and point weights, LN2 the next block's q|k|v and out weights.  The two
+    // chains each read their share.  The inverted-FFN weights are left cold:
     // warming them measured no gain.
     sana::CacheWarm warm1, warm2;
     {
-        const int64_t parts = Btot > B ? Btot : 1, part = Btot > B ? b0 : 0;
+        const int64_t parts = Btot / B, part = b0 / B;
         auto add = [&](sana::CacheWarm & cw, const DevMem & m) {
             const int64_t n16 = (int64_t)(m.bytes / 16), per = (n16 + parts - 1) / parts;
             const int64_t lo = std::min(n16, per * part), hi = std::min(n16, lo + per);
@@ -528,7 +510,7 @@ void enqueue_block(sana_dit * c, int64_t i, int64_t B, int64_t N, const float * 
                                    w.has_ln1 ? w.ln1_g.as<float>() : nullptr, w.has_ln1 ? w.ln1_b.as<float>() : nullptr,
                                    mod, nullptr, 6 * C, 0, C, s, &warm1),
                  "ln_modulate");
-    float * la_ws = (b0 > 0 && B == 1) ? c->la_ws2.as<float>() : c->la_ws.as<float>();
+    float * la_ws = b0 > 0 ? c->la_ws2.as<float>() : c->la_ws.as<float>();
     if (qkv_split_layout(c, N)) {
         half_t * kt16 = c->la_kt.as<half_t>() + b0 * C * N;
         half_t * vt16 = c->la_vt.as<half_t>() + b0 * C * N;
@@ -595,27 +577,113 @@ void join_from(hipEvent_t ev, hipStream_t s, hipStream_t s2) {
     hip_check(hipStreamWaitEvent(s, ev, 0), "hipStreamWaitEvent");
 }
 
-void enqueue_body(sana_dit * c, int64_t Bl, int64_t Hh, int64_t Ww, const float * xbias, float * out,
-                  hipStream_t s);
+// Whether the batch runs as two concurrent chains of blocks (the unconditional
+// and the conditional half): each kernel then covers half the rows, and the
+// chains fill each other's launch gaps and tails and share the weights through
+// the caches.
+int64_t chain_count(const sana_dit * c, int64_t B) { return c->cfg_branches && B % 2 == 0 ? 2 : 1; }
+
+// Capture `body` on the context stream into an executable graph.
+template <class Body>
+hipGraphExec_t capture_graph(sana_dit * c, Body body) {
+    hipGraph_t g = nullptr;
+    hip_check(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+    try {
+        body(c->stream);
+    } catch (...) {
+        (void)hipStreamEndCapture(c->stream, &g);
+        if (g) (void)hipGraphDestroy(g);
+        throw;
+    }
+    hip_check(hipStreamEndCapture(c->stream, &g), "hipStreamEndCapture");
+    hipGraphExec_t exec = nullptr;
+    hipError_t r = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    hip_check(r, "hipGraphInstantiate");
+    return exec;
+}
+
+// Chain k of n over all blocks as a cached graph of its own.
+hipGraphExec_t chain_graph(sana_dit * c, int64_t k, int64_t n, int64_t B, int64_t N, const float * xbias) {
+    const std::array<int64_t, 6> key = {k, n, B, N, c->ctx_L, xbias != nullptr};
+    auto it = c->graphs.find(key);
+    if (it == c->graphs.end()) {
+        if (c->graphs.size() >= 64) {  // bounded: callers rarely use this many shapes
+            hip_check(hipStreamSynchronize(c->stream), "graph cache");
+            hip_check(hipStreamSynchronize(c->stream2), "graph cache");
+            drop_graphs(c);
+        }
+        const int64_t rows = B / n;
+        hipGraphExec_t e = capture_graph(c, [&](hipStream_t s) {
+            for (int64_t i = 0; i < c->L_; ++i)
+                enqueue_block(c, i, rows, N, xbias, s, nullptr, nullptr, k * rows, B, (int)n);
+        });
+        it = c->graphs.emplace(key, e).first;
+    }
+    return it->second;
+}
+
+// Every block on x32, ordered on s.  Two chains are two linear graphs on two
+// streams, forked before the first block and joined after the last.  As two
+// branches of one graph (which it replaces) each pair of nodes cost the host
+// 5.2 us per launch, 1.6 ms in all, against 0.2 ms for two linear graphs: the
+// 512 px step 3.60 -> 3.36 ms in a row and 4.45 -> 3.56 ms alone, the 1024 px
+// step 6.47 -> 5.73 ms alone.  Direct launches cost 4 us of host time each.
+// Chain 0 runs on s itself: a third stream that waits for the pair slows every
+// kernel of both by 1 us while its wait is queued.  xbias is the context's own
+// mask buffer or null.  `direct`: kernel launches instead of graphs.
+void run_all_blocks(sana_dit * c, int64_t B, int64_t N, const float * xbias, hipStream_t s, bool direct) {
+    const int64_t n = chain_count(c, B);
+    if (n == 1) {
+        if (direct)
+            for (int64_t i = 0; i < c->L_; ++i) enqueue_block(c, i, B, N, xbias, s);
+        else
+            hip_check(hipGraphLaunch(chain_graph(c, 0, 1, B, N, xbias), s), "hipGraphLaunch");
+        return;
+    }
+    hipGraphExec_t g[2] = {nullptr, nullptr};
+    if (!direct)
+        for (int64_t k = 0; k < 2; ++k) g[k] = chain_graph(c, k, 2, B, N, xbias);
+    fork_to(c->ev_fork, s, c->stream2);
+    if (direct) {
+        for (int64_t i = 0; i < c->L_; ++i)
+            for (int64_t k = 0; k < 2; ++k)
+                enqueue_block(c, i, B / 2, N, xbias, k ? c->stream2 : s, nullptr, nullptr, k * (B / 2), B, 2);
+    } else {
+        hip_check(hipGraphLaunch(g[0], s), "hipGraphLaunch");
+        hip_check(hipGraphLaunch(g[1], c->stream2), "hipGraphLaunch");
+    }
+    join_from(c->ev_join, s, c->stream2);
+}
+
+// The blocks and the final layer.
+void enqueue_body(sana_dit * c, int64_t Bl, int64_t N, const float * xbias, float * out, hipStream_t s, bool direct) {
+    const int64_t B = 2 * Bl;
+    run_all_blocks(c, B, N, xbias, s, direct);
+    launch_check(sana::final_layer(c->x32.as<float>(), c->emb.as<float>(), c->sst_final.as<float>(),
+                                   c->w_proj.as<float>(), c->b_proj.as<float>(), c->fin32.as<float>(), out, (int)B,
+                                   (int)N, (int)c->C, (int)c->Cl, 1e-6f, s),
+                 "final_layer");
+}
 
 // The forward: patch and time embeddings, then the blocks and the final layer.
 // (Running the patch embedding on the second stream beside the time embedding
 // measured no faster.)
-void enqueue_forward(sana_dit * c, const float * latent, int64_t Bl, int64_t Hh, int64_t Ww, const float * xbias,
-                     float * out, hipStream_t s) {
-    enqueue_patch_embed(c, latent, Bl, Hh * Ww, s);
+void enqueue_forward(sana_dit * c, const float * latent, int64_t Bl, int64_t N, const float * xbias, float * out,
+                     hipStream_t s, bool direct) {
+    enqueue_patch_embed(c, latent, Bl, N, s);
     enqueue_time(c, 2 * Bl, s);
-    enqueue_body(c, Bl, Hh, Ww, xbias, out, s);
+    enqueue_body(c, Bl, N, xbias, out, s, direct);
 }
 
 // The step: the caption projection and cross K/V on s, and beside them on the
 // second stream the forward's head (patch and time embeddings), which needs
 // neither; the blocks start when both are done (step 5.564 -> 5.518 ms in one
 // process; the head's ~60 us of small kernels hide behind the context GEMMs).
-void enqueue_step(sana_dit * c, const float * caption, int64_t L, const float * latent, int64_t Bl, int64_t Hh,
-                  int64_t Ww, const float * xbias, float * out, hipStream_t s) {
+void enqueue_step(sana_dit * c, const float * caption, int64_t L, const float * latent, int64_t Bl, int64_t N,
+                  const float * xbias, float * out, hipStream_t s, bool direct) {
     fork_to(c->ev_head_fork, s, c->stream2);
-    enqueue_patch_embed(c, latent, Bl, Hh * Ww, c->stream2);
+    enqueue_patch_embed(c, latent, Bl, N, c->stream2);
     enqueue_time(c, 2 * Bl, c->stream2);
     enqueue_context_rows(c, caption, false, 2 * Bl, L, s);
     // cross K on s and cross V^T on the second stream (after the head)
@@ -623,35 +691,16 @@ void enqueue_step(sana_dit * c, const float * caption, int64_t L, const float * 
     enqueue_context_k(c, 2 * Bl, L, s);
     enqueue_context_vt(c, 2 * Bl, L, c->stream2);
     join_from(c->ev_head_join, s, c->stream2);
-    enqueue_body(c, Bl, Hh, Ww, xbias, out, s);
+    enqueue_body(c, Bl, N, xbias, out, s, direct);
 }
 
-// Blocks (the CFG pair as two concurrent chains) and the final layer.
-void enqueue_body(sana_dit * c, int64_t Bl, int64_t Hh, int64_t Ww, const float * xbias, float * out,
-                  hipStream_t s) {
-    const int64_t B = 2 * Bl, N = Hh * Ww;
-    // The CFG pair runs its two batch rows as two concurrent chains (graph
-    // branches): each kernel then covers half the rows, and the two chains fill
-    // each other's launch gaps and tails and share the weights through the caches.
-    if (B == 2 && c->cfg_branches) {
-        // batch row 0 on s, row 1 on stream2, forked after the time embedding
-        // and joined before the final layer
-        hip_check(hipEventRecord(c->ev_fork, s), "hipEventRecord");
-        hip_check(hipStreamWaitEvent(c->stream2, c->ev_fork, 0), "hipStreamWaitEvent");
-        for (int64_t i = 0; i < c->L_; ++i) {
-            enqueue_block(c, i, 1, N, xbias, s, nullptr, nullptr, 0, 2, 2);
-            enqueue_block(c, i, 1, N, xbias, c->stream2, nullptr, nullptr, 1, 2, 2);
-        }
-        hip_check(hipEventRecord(c->ev_join, c->stream2), "hipEventRecord");
-        hip_check(hipStreamWaitEvent(s, c->ev_join, 0), "hipStreamWaitEvent");
-    } else {
-        for (int64_t i = 0; i < c->L_; ++i) enqueue_block(c, i, B, N, xbias, s);
-    }
-    launch_check(sana::final_layer(c->x32.as<float>(), c->emb.as<float>(), c->sst_final.as<float>(),
-                                   c->w_proj.as<float>(), c->b_proj.as<float>(), c->fin32.as<float>(), out, (int)B,
-                                   (int)N, (int)c->C,
-                                   (int)c->Cl, 1e-6f, s),
-                 "final_layer");
+// Whether work on s is launched kernel by kernel: with graphs off, and while
+// the caller captures s (it then becomes part of the caller's graph).
+bool direct_launches(const sana_dit * c, hipStream_t s) {
+    if (!c->use_graphs) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (s != c->stream) hip_check(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing");
+    return cap != hipStreamCaptureStatusNone;
 }
 
 // Tensors every block needs (load_block_weights, src/transformer.cpp:214-308).
@@ -703,51 +752,6 @@ void set_t(sana_dit * c, int64_t B, float t, hipStream_t s) {
     hip_check(hipGetLastError(), "fill");
 }
 
-
-// Capture `body` on the context stream into an executable graph.
-template <class Body>
-hipGraphExec_t capture_graph(sana_dit * c, Body body) {
-    hipGraph_t g = nullptr;
-    hip_check(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    try {
-        body(c->stream);
-    } catch (...) {
-        (void)hipStreamEndCapture(c->stream, &g);
-        if (g) (void)hipGraphDestroy(g);
-        throw;
-    }
-    hip_check(hipStreamEndCapture(c->stream, &g), "hipStreamEndCapture");
-    hipGraphExec_t exec = nullptr;
-    hipError_t r = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    hip_check(r, "hipGraphInstantiate");
-    return exec;
-}
-
-template <class T>
-void key_append(std::string & k, const T & v) {
-    k.append(reinterpret_cast<const char *>(&v), sizeof(T));
-}
-
-// Run `body` on stream s through a cached HIP graph (captured on the context
-// stream on first use for this key).
-template <class Body>
-void run_graph(sana_dit * c,
-               const std::tuple<int, int64_t, int64_t, int64_t, int64_t, const void *, const void *, const void *,
-                                const void *> & key,
-               hipStream_t s, Body body) {
-    if (!c->use_graphs) {
-        body(s);
-        return;
-    }
-    auto it = c->graphs.find(key);
-    if (it == c->graphs.end()) {
-        GraphEntry e;
-        e.exec = capture_graph(c, body);
-        it = c->graphs.emplace(key, e).first;
-    }
-    hip_check(hipGraphLaunch(it->second.exec, s), "hipGraphLaunch");
-}
 
 struct BlockSuffix {
     const char * name;
@@ -1429,11 +1433,8 @@ int sana_dit_forward_device(sana_dit * c, const float * d_latent, int64_t Bl, in
         c->last_B = B;
         c->last_N = N;
         set_t(c, B, t, s);
-        run_graph(c, std::make_tuple(1, Bl, Hh, Ww, c->ctx_L, (const void *)d_latent, (const void *)d_out,
-                                     (const void *)nullptr, (const void *)(intptr_t)c->ctx_bias),
-                  s, [&](hipStream_t gs) {
-                      enqueue_forward(c, d_latent, Bl, Hh, Ww, c->ctx_bias ? c->bias.as<float>() : nullptr, d_out, gs);
-                  });
+        enqueue_forward(c, d_latent, Bl, N, c->ctx_bias ? c->bias.as<float>() : nullptr, d_out, s,
+                        direct_launches(c, s));
     });
 }
 
@@ -1472,13 +1473,13 @@ int sana_dit_step_device(sana_dit * c, const float * d_caption, int64_t L, const
         c->last_B = B;
         c->last_N = N;
         set_t(c, B, t, s);
-        run_graph(c, std::make_tuple(2, Bl, Hh, Ww, L, (const void *)d_caption, (const void *)d_bias,
-                                     (const void *)d_latent, (const void *)d_out),
-                  s, [&](hipStream_t gs) { enqueue_step(c, d_caption, L, d_latent, Bl, Hh, Ww, d_bias, d_out, gs); });
-        // keep the context state consistent for later sana_dit_forward* calls
+        // the mask goes to the context's buffer, where the blocks (and later
+        // sana_dit_forward* calls) read it
         c->ctx_bias = d_bias != nullptr;
         if (d_bias)
             hip_check(hipMemcpyAsync(c->bias.p, d_bias, (size_t)B * L * 4, hipMemcpyDeviceToDevice, s), "bias");
+        enqueue_step(c, d_caption, L, d_latent, Bl, N, d_bias ? c->bias.as<float>() : nullptr, d_out, s,
+                     direct_launches(c, s));
         c->ctx_ready = true;
     });
 }
@@ -1545,10 +1546,7 @@ float flow_lambda(float sigma) {  // log(alpha) - log(sigma) with alpha = 1 - si
 
 // The whole loop on `s`: step i runs the forward at timesteps[i] on latent
 // buffer i % 2 and writes buffer (i + 1) % 2; the converted outputs of the two
-// latest steps alternate in loop_x0.  With graphs on, the whole loop (latent
-// copy, and per step the timestep fill, the forward and the CFG + solver
-// update) is one graph, captured once per shape, buffers and schedule.
-// Returns the buffer holding the result.
+// latest steps alternate in loop_x0.  Returns the buffer holding the result.
 float * enqueue_loop(sana_dit * c, const float * d_latent, int64_t Bl, int64_t Hh, int64_t Ww, const float * ts,
                      const float * sg, int64_t steps, float guidance, hipStream_t s) {
     const int64_t n = Bl * c->Cl * Hh * Ww;
@@ -1561,53 +1559,31 @@ float * enqueue_loop(sana_dit * c, const float * d_latent, int64_t Bl, int64_t H
     c->last_B = B;
     c->last_N = N;
     const float * xbias = c->ctx_bias ? c->bias.as<float>() : nullptr;
-    auto body = [&](hipStream_t gs) {
-        hip_check(hipMemcpyAsync(c->loop_lat[0].p, d_latent, (size_t)n * 4, hipMemcpyDeviceToDevice, gs), "latent");
-        for (int64_t i = 0; i < steps; ++i) {
-            float * cur = c->loop_lat[i & 1].as<float>();
-            float * nxt = c->loop_lat[(i + 1) & 1].as<float>();
-            set_t(c, B, ts[i], gs);
-            enqueue_forward(c, cur, Bl, Hh, Ww, xbias, c->np_out.as<float>(), gs);
-            // step_sana_scheduler (src/scheduler.cpp:272-318) with solver_order 2, midpoint,
-            // lower_order_final: first order at the first and at the last step.
-            const bool first = i == 0 || i == steps - 1;
-            const float st_v = sg[i + 1], s0_v = sg[i];
-            const float alpha_t = 1.0f - st_v;
-            const float h = flow_lambda(st_v) - flow_lambda(s0_v);
-            const float ca = st_v / s0_v, cb = -alpha_t * (std::exp(-h) - 1.0f);
-            float cc = 0.0f, inv_r0 = 0.0f;
-            if (!first) {
-                const float h0 = flow_lambda(s0_v) - flow_lambda(sg[i - 1]);
-                inv_r0 = 1.0f / (h0 / h);
-                cc = -0.5f * alpha_t * (std::exp(-h) - 1.0f);
-            }
-            hipLaunchKernelGGL(cfg_dpm_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, gs,
-                               c->np_out.as<float>(), cur, c->loop_x0[(i + 1) & 1].as<float>(), nxt,
-                               c->loop_x0[i & 1].as<float>(), (int)n, guidance, s0_v, ca, cb, cc, inv_r0,
-                               first ? 0 : 1);
-            hip_check(hipGetLastError(), "cfg_dpm");
+    const bool direct = direct_launches(c, s);
+    hip_check(hipMemcpyAsync(c->loop_lat[0].p, d_latent, (size_t)n * 4, hipMemcpyDeviceToDevice, s), "latent");
+    for (int64_t i = 0; i < steps; ++i) {
+        float * cur = c->loop_lat[i & 1].as<float>();
+        float * nxt = c->loop_lat[(i + 1) & 1].as<float>();
+        set_t(c, B, ts[i], s);
+        enqueue_forward(c, cur, Bl, N, xbias, c->np_out.as<float>(), s, direct);
+        // step_sana_scheduler (src/scheduler.cpp:272-318) with solver_order 2, midpoint,
+        // lower_order_final: first order at the first and at the last step.
+        const bool first = i == 0 || i == steps - 1;
+        const float st_v = sg[i + 1], s0_v = sg[i];
+        const float alpha_t = 1.0f - st_v;
+        const float h = flow_lambda(st_v) - flow_lambda(s0_v);
+        const float ca = st_v / s0_v, cb = -alpha_t * (std::exp(-h) - 1.0f);
+        float cc = 0.0f, inv_r0 = 0.0f;
+        if (!first) {
+            const float h0 = flow_lambda(s0_v) - flow_lambda(sg[i - 1]);
+            inv_r0 = 1.0f / (h0 / h);
+            cc = -0.5f * alpha_t * (std::exp(-h) - 1.0f);
         }
-    };
-    if (!c->use_graphs) {
-        body(s);
-    } else {
-        std::string key;
-        for (int64_t v : {Bl, Hh, Ww, c->ctx_L, (int64_t)c->ctx_bias, steps}) key_append(key, v);
-        for (const void * p : {(const void *)d_latent, (const void *)c->loop_lat[0].p, (const void *)c->loop_lat[1].p,
-                               (const void *)c->loop_x0[0].p, (const void *)c->loop_x0[1].p,
-                               (const void *)c->np_out.p})
-            key_append(key, p);
-        key_append(key, guidance);
-        for (int64_t i = 0; i < steps; ++i) key_append(key, ts[i]);
-        for (int64_t i = 0; i <= steps; ++i) key_append(key, sg[i]);
-        auto it = c->loop_graphs.find(key);
-        if (it == c->loop_graphs.end()) {
-            if (c->loop_graphs.size() >= 4) drop_loop_graphs(c);
-            GraphEntry e;
-            e.exec = capture_graph(c, body);
-            it = c->loop_graphs.emplace(key, e).first;
-        }
-        hip_check(hipGraphLaunch(it->second.exec, s), "hipGraphLaunch");
+        hipLaunchKernelGGL(cfg_dpm_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                           c->np_out.as<float>(), cur, c->loop_x0[(i + 1) & 1].as<float>(), nxt,
+                           c->loop_x0[i & 1].as<float>(), (int)n, guidance, s0_v, ca, cb, cc, inv_r0,
+                           first ? 0 : 1);
+        hip_check(hipGetLastError(), "cfg_dpm");
     }
     hip_check(hipEventRecord(c->ev_loop, s), "hipEventRecord");
     c->loop_steps = steps;
@@ -1703,11 +1679,11 @@ int sana_dit_time_kernel(sana_dit * c, int which, int iters, float * avg_ms, dou
     if (which < 0 || which > 9) return set_err(SANA_ERR_INVALID_ARGUMENT, "which must be 0..9");
     if (!c->ctx_ready) return set_err(SANA_ERR_STATE, "no context set");
     return guarded([&] {
-        // The shape and launch of the last forward: one batch row per launch
-        // (co = 2) when the CFG pair ran as two branches, else the whole batch.
+        // The shape and launch of the last forward: half the batch per launch
+        // (co = 2) when it ran as two chains, else the whole batch.
         const int64_t N = c->last_N, C = c->C, E = c->E, F = c->F, Lc = c->ctx_L, Btot = c->last_B;
-        const bool branches = Btot == 2 && c->cfg_branches;
-        const int64_t B = branches ? 1 : Btot, M = B * N, side = (int64_t)std::llround(std::sqrt((double)N));
+        const bool branches = chain_count(c, Btot) == 2;
+        const int64_t B = branches ? Btot / 2 : Btot, M = B * N, side = (int64_t)std::llround(std::sqrt((double)N));
         const int co = branches ? 2 : 1;
         hipStream_t s = c->stream;
         const float * xbias = c->ctx_bias ? c->bias.as<float>() : nullptr;

@@ -381,3 +381,48 @@ def test_small_forward_fewer_tokens_more_chunks(small_model):
     d.set_context(caption, projected=False)
     d.forward(lat33, 999.0)
     assert np.array_equal(d.forward(lat31, 999.0), ref)
+
+
+@pytest.mark.parametrize("images,masked", [(1, True), (2, False)])
+def test_small_step_streams_buffers_and_capture(small_model, images, masked):
+    """One step on the context's stream, on a caller's stream with fresh
+    buffers (the cached block chains hold none of the caller's), and captured
+    into a caller's graph (replayed on new contents with eager steps between):
+    all bit-identical."""
+    import torch
+    m, d = small_model
+    dev = torch.device("cuda:0")
+    shape = (images, 8, 8, 8)
+
+    def data(seed):
+        cap = torch.from_numpy(O.randn((2 * images, 16, 96), seed)).to(dev)
+        lat = torch.from_numpy(O.randn(shape, seed + 1)).to(dev)
+        bias = torch.zeros((2 * images, 16), device=dev)
+        bias[:, 9:] = -10000.0
+        return cap, lat, bias if masked else None
+
+    def step(x, stream=None):
+        out = torch.empty((2 * images, 8, 8, 8), device=dev)
+        torch.cuda.synchronize()
+        d.step_device(x[0], 16, x[2], x[1], shape, 999.0, out, stream.cuda_stream if stream else None)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    refs = [step(data(s)) for s in (61, 71, 81)]
+    user = torch.cuda.Stream()
+    for s, ref in zip((61, 71, 81), refs):
+        assert np.array_equal(step(data(s), user), ref)
+    x, out = data(61), torch.empty((2 * images, 8, 8, 8), device=dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=user):
+        d.step_device(x[0], 16, x[2], x[1], shape, 999.0, out, user.cuda_stream)
+    for s, ref in list(zip((61, 71, 81), refs)) * 2:
+        y = data(s)
+        x[0].copy_(y[0])
+        x[1].copy_(y[1])
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), ref)
+        assert np.array_equal(step(data(71)), refs[1])
