@@ -58,7 +58,7 @@ constexpr int kTK = 32;
 // VA, VB: floats per global load of A and B, 4 where base, strides and extents
 // are multiples of 4 elements (16 bytes), else 1.
 //
-// Measured on MI355X: 2048 x 1152 x 1152 77 us (71 TFLOP/s); with the other
+// Measured on MI355X: 2048 x 1152 x 1152 65 us (84 TFLOP/s); with the other
 // kernels of this file the fp32 self-attention block (2 x 1024 tokens, four
 // such products) went from 1316 to 314 us and the cross-attention block (2 x
 // 256 tokens, 300 keys) from 787 to 140 us, against a 64 x 64 tile with
@@ -708,16 +708,20 @@ int sana_op_gemm_f32(const float * A, int64_t lda, int64_t strideA, const float 
     const bool va = aligned16(A) && lda % 4 == 0 && K % 4 == 0 && (batch == 1 || strideA % 4 == 0);
     const bool vb = aligned16(B) && ldb % 4 == 0 && (b_transposed ? K : N) % 4 == 0 && (batch == 1 || strideB % 4 == 0);
     p.vec_c = aligned16(C) && ldc % 4 == 0 && (batch == 1 || strideC % 4 == 0);
-    // The tile whose busiest CU has the least area to multiply (the matrix rate
-    // bounds every shape here; ties go to the larger tile, which reads less).
+    // The tile with the least modelled time: `fixed` + `round` per round of 256
+    // workgroups, both measured at K = 1152 (us x 10; 64 to 16384 rows, 1152
+    // columns, within 10 %).  Small tiles have the shorter k-step chain, large
+    // ones fewer LDS reads per product.  2048 x 1152: 32x32 72 us, 64x32 65, 64x96
+    // 73; 512 rows 27, 31, 44; 4096 rows 129, 111, 103; 64 products of 4096 x 72
+    // x 300: 203, 181, 164 (64x64 and 32x64 lie within 1 % of these three).
     struct {
-        int64_t m, n;
-    } const tiles[3] = {{64, 64}, {32, 64}, {32, 32}};
+        int64_t m, n, round, fixed;
+    } const tiles[3] = {{64, 96, 304, 125}, {64, 32, 110, 105}, {32, 32, 70, 90}};
     int best = 0;
     int64_t best_cost = INT64_MAX;
     for (int i = 0; i < 3; ++i) {
         const int64_t t = ((M + tiles[i].m - 1) / tiles[i].m) * ((N + tiles[i].n - 1) / tiles[i].n) * batch;
-        const int64_t cost = (t + 255) / 256 * tiles[i].m * tiles[i].n;
+        const int64_t cost = tiles[i].fixed + (t + 255) / 256 * tiles[i].round;
         if (t / batch <= INT32_MAX && cost < best_cost) {
             best = i;
             best_cost = cost;
@@ -725,8 +729,8 @@ int sana_op_gemm_f32(const float * A, int64_t lda, int64_t strideA, const float 
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bt = b_transposed != 0;
-    if (best == 0) launch_gemm_f32<64, 64>(p, bt, va, vb, (unsigned)batch, s);
-    else if (best == 1) launch_gemm_f32<32, 64>(p, bt, va, vb, (unsigned)batch, s);
+    if (best == 0) launch_gemm_f32<64, 96>(p, bt, va, vb, (unsigned)batch, s);
+    else if (best == 1) launch_gemm_f32<64, 32>(p, bt, va, vb, (unsigned)batch, s);
     else launch_gemm_f32<32, 32>(p, bt, va, vb, (unsigned)batch, s);
     return launched("gemm_f32");
 }
