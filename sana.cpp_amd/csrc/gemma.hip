@@ -7,9 +7,9 @@
 //   a16  = rmsnorm(x) * attn_norm                        gemma_norm_kernel
 //   qkv  = a16 [Wq; Wk; Wv]^T                            one MFMA GEMM, fp32 out
 //   q16, k16 = rope(q) * query_scale, rope(k); V^T       gemma_qkv_kernel
-//   S_h  = q16_h k16_kv(h)^T                             all heads in one batched GEMM
-//   P_h  = softmax(causal / window mask, soft-cap)       gemma_softmax_kernel
-//   o16_h = P_h V_kv(h)                                  all heads in one batched GEMM (B = V^T)
+//   o16_h = softmax(mask(softcap(q16_h k16_kv(h)^T))) V_kv(h)
+//                                                        gemma_attention_kernel, all sequences and heads;
+//                                                        d other than 64, 128, 256: attention_by_products
 //   x   += rmsnorm(o16 Wo^T) * post_attention_norm       split-K GEMM + gemma_norm_kernel
 //   a16  = rmsnorm(x) * ffn_norm
 //   g16  = gelu_tanh(a16 Wgate^T) * (a16 Wup^T)        one GEMM, gate / up rows
@@ -39,6 +39,8 @@
 using sana::half_t;
 using namespace sana_host;
 
+#define SANA_LDS(p) ((__attribute__((address_space(3))) void *)(p))
+
 namespace {
 
 unsigned blocks_for(int64_t n, int per = 256) { return (unsigned)((n + per - 1) / per); }
@@ -53,34 +55,44 @@ __global__ void gemma_embed_kernel(const int32_t * __restrict__ tok, const f16 *
 }
 
 // One workgroup of 256 threads per row of C (<= 1024 * NC4) channels:
-// v = y / sqrt(mean(y^2) + eps) * w, y the fixed-order sum of `parts` split-K
+// v = y / sqrt(mean(y^2) + eps) * w, y the fixed-order sum of PARTS split-K
 // partials part_stride floats apart; the sum of squares is reduced over the
-// four waves through LDS.  mode 0: out16 = fp16(v); 1: x += v (post-norm
+// four waves through LDS.  MODE 0: out16 = fp16(v); 1: x += v (post-norm
 // residual, out32 = x); 2: out32 = v; 3: x += v as mode 1, then the next
 // pre-norm of the new row, out16 = fp16(x / sqrt(mean(x^2) + eps) * w2), with
 // the same summation order as a separate mode-0 launch on x.
-template <int NC4>
-__global__ __launch_bounds__(256) void gemma_norm_kernel(const float * __restrict__ y, int parts,
-                                                         int64_t part_stride, int C, int M,
-                                                         const float * __restrict__ w, float eps, int mode,
+// Every load of the row (partials, residual, weights) is requested before the
+// first sum, without branches (columns past C read the last one and count as
+// zero): one memory latency instead of four in a row (23 rows of 2304, four
+// partials, modes 1 and 3: 7.4 -> 4.75 us; 738 rows, two partials: 9.87 -> 8.6).
+template <int NC4, int MODE, int PARTS>
+__global__ __launch_bounds__(256) void gemma_norm_kernel(const float * __restrict__ y, int64_t part_stride, int C,
+                                                         const float * __restrict__ w, float eps,
                                                          f16 * __restrict__ out16, float * __restrict__ out32,
                                                          const float * __restrict__ w2) {
-    __shared__ float wsum[4];
+    __shared__ float wsum[8];
     const int row = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63;
     const int n4 = C >> 2;
-    const float4 * yr = reinterpret_cast<const float4 *>(y + (int64_t)row * C);
-    float4 v[NC4];
+    float4 v[NC4], u[PARTS][NC4], g[NC4], g2[MODE == 3 ? NC4 : 1], x[MODE == 1 || MODE == 3 ? NC4 : 1];
+#pragma unroll
+    for (int i = 0; i < NC4; ++i) {
+        const int c4 = min(tid + 256 * i, n4 - 1);
+#pragma unroll
+        for (int z = 0; z < PARTS; ++z)
+            u[z][i] = reinterpret_cast<const float4 *>(y + z * part_stride + (int64_t)row * C)[c4];
+        if constexpr (MODE == 1 || MODE == 3) x[i] = reinterpret_cast<const float4 *>(out32 + (int64_t)row * C)[c4];
+        g[i] = reinterpret_cast<const float4 *>(w)[c4];
+        if constexpr (MODE == 3) g2[i] = reinterpret_cast<const float4 *>(w2)[c4];
+    }
     float ss = 0.0f;
 #pragma unroll
     for (int i = 0; i < NC4; ++i) {
-        const int c4 = tid + 256 * i;
-        v[i] = c4 < n4 ? yr[c4] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (int z = 1; z < parts; ++z) {
-            if (c4 >= n4) break;
-            const float4 u = reinterpret_cast<const float4 *>(y + z * part_stride + (int64_t)row * C)[c4];
-            v[i] = make_float4(v[i].x + u.x, v[i].y + u.y, v[i].z + u.z, v[i].w + u.w);
-        }
+        v[i] = u[0][i];
+#pragma unroll
+        for (int z = 1; z < PARTS; ++z)
+            v[i] = make_float4(v[i].x + u[z][i].x, v[i].y + u[z][i].y, v[i].z + u[z][i].z, v[i].w + u[z][i].w);
+        if (tid + 256 * i >= n4) v[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         ss += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
     }
     ss = wave_sum(ss);
@@ -93,18 +105,16 @@ __global__ __launch_bounds__(256) void gemma_norm_kernel(const float * __restric
     for (int i = 0; i < NC4; ++i) {
         const int c4 = tid + 256 * i;
         if (c4 >= n4) continue;
-        const float4 g = reinterpret_cast<const float4 *>(w)[c4];
-        float o[4] = {v[i].x * inv * g.x, v[i].y * inv * g.y, v[i].z * inv * g.z, v[i].w * inv * g.w};
-        if (mode == 0) {
+        float o[4] = {v[i].x * inv * g[i].x, v[i].y * inv * g[i].y, v[i].z * inv * g[i].z, v[i].w * inv * g[i].w};
+        if constexpr (MODE == 0) {
             f16x4 h;
 #pragma unroll
             for (int e = 0; e < 4; ++e) h[e] = (f16)o[e];
             *reinterpret_cast<f16x4 *>(out16 + (int64_t)row * C + 4 * c4) = h;
         } else {
             float4 * xr = reinterpret_cast<float4 *>(out32 + (int64_t)row * C) + c4;
-            if (mode == 1 || mode == 3) {
-                const float4 x = *xr;
-                const float4 xn = make_float4(x.x + o[0], x.y + o[1], x.z + o[2], x.w + o[3]);
+            if constexpr (MODE == 1 || MODE == 3) {
+                const float4 xn = make_float4(x[i].x + o[0], x[i].y + o[1], x[i].z + o[2], x[i].w + o[3]);
                 *xr = xn;
                 v[i] = xn;  // the new residual row, for mode 3's second norm
                 ss2 += (xn.x * xn.x + xn.y * xn.y) + (xn.z * xn.z + xn.w * xn.w);
@@ -113,62 +123,354 @@ __global__ __launch_bounds__(256) void gemma_norm_kernel(const float * __restric
             }
         }
     }
-    if (mode != 3) return;
-    ss2 = wave_sum(ss2);
-    __syncthreads();  // every wave has read wsum
-    if (lane == 0) wsum[tid >> 6] = ss2;
-    __syncthreads();
-    const float tot2 = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-    const float inv2 = 1.0f / sqrtf(tot2 / (float)C + eps);
+    if constexpr (MODE == 3) {
+        ss2 = wave_sum(ss2);
+        if (lane == 0) wsum[4 + (tid >> 6)] = ss2;
+        __syncthreads();
+        const float tot2 = (wsum[4] + wsum[5]) + (wsum[6] + wsum[7]);
+        const float inv2 = 1.0f / sqrtf(tot2 / (float)C + eps);
 #pragma unroll
-    for (int i = 0; i < NC4; ++i) {
-        const int c4 = tid + 256 * i;
-        if (c4 >= n4) continue;
-        const float4 g = reinterpret_cast<const float4 *>(w2)[c4];
-        f16x4 h;
-        h[0] = (f16)(v[i].x * inv2 * g.x);
-        h[1] = (f16)(v[i].y * inv2 * g.y);
-        h[2] = (f16)(v[i].z * inv2 * g.z);
-        h[3] = (f16)(v[i].w * inv2 * g.w);
-        *reinterpret_cast<f16x4 *>(out16 + (int64_t)row * C + 4 * c4) = h;
+        for (int i = 0; i < NC4; ++i) {
+            const int c4 = tid + 256 * i;
+            if (c4 >= n4) continue;
+            f16x4 h;
+            h[0] = (f16)(v[i].x * inv2 * g2[i].x);
+            h[1] = (f16)(v[i].y * inv2 * g2[i].y);
+            h[2] = (f16)(v[i].z * inv2 * g2[i].z);
+            h[3] = (f16)(v[i].w * inv2 * g2[i].w);
+            *reinterpret_cast<f16x4 *>(out16 + (int64_t)row * C + 4 * c4) = h;
+        }
     }
 }
 
-// qkv32 [T][(nh + 2 nkv) d] -> q16 [T][nh d] = rope(q) * qscale, k16 [T][nkv d]
-// = rope(k), vt16 [nkv][d][Tp] = V^T (tokens T..Tp-1 zero).  NeoX RoPE: pair
-// (i, i + d/2) of a head rotated by t * theta^(-2i/d).  One thread per
-// (token, rotation pair) of the q and k heads, and per (token, channel) of v.
-__global__ void gemma_qkv_kernel(const float * __restrict__ qkv, int T, int Tp, int nh, int nkv, int d,
-                                 float theta, float qscale, f16 * __restrict__ q16, f16 * __restrict__ k16,
-                                 f16 * __restrict__ vt16) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// s_waitcnt with only the vector-memory (or only the LDS) counter constrained;
+// the scheduler moves no memory operation across.
+template <int N>
+__device__ inline void wait_vmcnt() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ inline void wait_lgkmcnt0() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The sequences of one encode as the kernels see them (sana_gemma_encode_pair
+// has two): rows [row0, row0 + T) of the token-major buffers.
+struct GemmaSeqs {
+    int n;
+    int row0[2], T[2], Tp[2];
+    int64_t vt_off[2];
+};
+
+// qkv32 [M][(nh + 2 nkv) d] -> q16 [M][nh d] = rope(q) * qscale, k16 [M][nkv d]
+// = rope(k), vt16 [nkv][d][Tp] per sequence = V^T (tokens T..Tp-1 zero; `perm`:
+// within each 16 tokens in the order 0-3, 8-11, 4-7, 12-15, which
+// gemma_attention_kernel reads).  NeoX
+// RoPE: pair (i, i + d/2) of a head rotated by t * theta^(-2i/d), t the position
+// in its sequence.  The first rope_blocks workgroups take one (row, rotation
+// pair) per thread for four heads (one powf and sincosf instead of one per
+// head); the others transpose a 64 x 64 (token, channel) tile of V through
+// LDS, so both sides move whole lines (read along the tokens, each lane touched
+// a line of its own).  438 + 300 rows of 4096: 2 x 8.6 -> 6.5 us, one launch.
+__global__ __launch_bounds__(256) void gemma_qkv_kernel(const float * __restrict__ qkv, GemmaSeqs sq, int M, int nh,
+                                                        int nkv, int d, float theta, float qscale,
+                                                        int rope_blocks, int perm, f16 * __restrict__ q16,
+                                                        f16 * __restrict__ k16, f16 * __restrict__ vt16) {
     const int half = d / 2, ld = (nh + 2 * nkv) * d;
-    const int64_t nrot = (int64_t)T * (nh + nkv) * half;
-    if (i < nrot) {
-        const int t = (int)(i / ((nh + nkv) * half));
-        const int r = (int)(i - (int64_t)t * (nh + nkv) * half);
-        const int head = r / half, p = r - head * half;  // heads 0..nh-1 are q, then k
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x < rope_blocks) {
+        // (row, group of 4 heads, pair)
+        const int64_t i = (int64_t)blockIdx.x * 256 + tid;
+        const int groups = (nh + nkv + 3) / 4;
+        if (i >= (int64_t)M * groups * half) return;
+        const int rg = (int)(i / half), p = (int)(i - (int64_t)rg * half);
+        const int row = rg / groups, h0 = (rg - row * groups) * 4;
+        const int t = row - (sq.n > 1 && row >= sq.row0[1] ? sq.row0[1] : 0);
         const float inv = powf(theta, -2.0f * (float)p / (float)d);
         float sn, cs;
         sincosf((float)t * inv, &sn, &cs);
-        const float * src = qkv + (int64_t)t * ld + head * d;
-        const float a = src[p], b = src[p + half];
-        float oa = a * cs - b * sn, ob = b * cs + a * sn;
-        if (head < nh) {
-            f16 * dst = q16 + (int64_t)t * nh * d + head * d;
-            dst[p] = (f16)(oa * qscale);
-            dst[p + half] = (f16)(ob * qscale);
-        } else {
-            f16 * dst = k16 + (int64_t)t * nkv * d + (head - nh) * d;
-            dst[p] = (f16)oa;
-            dst[p + half] = (f16)ob;
+        const float * src = qkv + (int64_t)row * ld + p;
+        float a[4], b[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int head = min(h0 + e, nh + nkv - 1);
+            a[e] = src[head * d];
+            b[e] = src[head * d + half];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int head = h0 + e;  // heads 0..nh-1 are q, then k
+            if (head >= nh + nkv) break;
+            const float oa = a[e] * cs - b[e] * sn, ob = b[e] * cs + a[e] * sn;
+            f16 * dst = head < nh ? q16 + ((int64_t)row * nh + head) * d : k16 + ((int64_t)row * nkv + head - nh) * d;
+            const float sc = head < nh ? qscale : 1.0f;
+            dst[p] = (f16)(oa * sc);
+            dst[p + half] = (f16)(ob * sc);
         }
         return;
     }
-    const int64_t j = i - nrot;
-    if (j >= (int64_t)nkv * d * Tp) return;
-    const int t = (int)(j % Tp), ch = (int)(j / Tp);  // ch = kvhead * d + dim
-    vt16[j] = t < T ? (f16)qkv[(int64_t)t * ld + (nh + nkv) * d + ch] : (f16)0.0f;
+    __shared__ f16 tile[64][72];
+    const int ctiles = nkv * d / 64;
+    int b = (int)blockIdx.x - rope_blocks, si = 0;
+    if (b >= sq.Tp[0] / 64 * ctiles) {
+        b -= sq.Tp[0] / 64 * ctiles;
+        si = 1;
+    }
+    const int t0 = b / ctiles * 64, c0 = b % ctiles * 64, T = sq.T[si], Tp = sq.Tp[si];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int item = tid + 256 * k, t = item >> 4, c = (item & 15) * 4;
+        const int tt = min(t0 + t, T - 1);
+        const float4 v = *reinterpret_cast<const float4 *>(qkv + (int64_t)(sq.row0[si] + tt) * ld + (nh + nkv) * d +
+                                                           c0 + c);
+        const bool ok = t0 + t < T;
+        const int u = perm ? (t & ~12) | (t & 4) << 1 | (t & 8) >> 1 : t;
+        tile[c][u] = ok ? (f16)v.x : (f16)0.0f;
+        tile[c + 1][u] = ok ? (f16)v.y : (f16)0.0f;
+        tile[c + 2][u] = ok ? (f16)v.z : (f16)0.0f;
+        tile[c + 3][u] = ok ? (f16)v.w : (f16)0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int item = tid + 256 * k, c = item >> 3, t = (item & 7) * 8;
+        *reinterpret_cast<f16x8 *>(vt16 + sq.vt_off[si] + (int64_t)(c0 + c) * Tp + t0 + t) =
+            *reinterpret_cast<const f16x8 *>(&tile[c][t]);
+    }
+}
+
+// e^x for x <= 0 (0 for -inf, NaN for NaN) on v_exp_f32: the exponent's rounding
+// leaves a relative error of |x| 2^-24 on top of the instruction's 1 ulp, far
+// below the fp16 rounding of the probabilities.
+__device__ inline float exp_f32(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
+
+// tanh to a few ulp: below 1/4 its series to x^9 (the next term is 9e-9 of it),
+// above 1 - 2 / (e^2x + 1).  Against expf and tanhf, whose branches every lane
+// walks: attention of 438 + 300 tokens 27.1 -> 25.0 us, of 23 tokens 10.4 -> 8.0.
+__device__ inline float tanh_f32(float x) {
+    const float t = x * x;
+    const float poly = x + x * t * (-1.0f / 3 + t * (2.0f / 15 + t * (-17.0f / 315 + t * (62.0f / 2835))));
+    const float a = fabsf(x);
+    const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a * 2.88539008f) + 1.0f);
+    return a < 0.25f ? poly : copysignf(big, x);
+}
+
+// Causal soft-capped attention with a sliding window, one pass (online
+// softmax), for all sequences and heads in one launch: head dims D of 64, 128
+// and 256 (others take attention_by_products: the score product, the softmax
+// and the P.V product, 56 us for 438 + 300 tokens of 8 heads of 256).
+// s = cap * tanh(q.k / cap) over keys j <= t (and j > t - window when
+// window > 0).
+//
+// A workgroup takes 32 queries of one head; its four waves take every fourth
+// block of 32 keys each, with a running max, sum and output of their own, which
+// are merged through LDS at the end: no barrier in the loop.  Each wave stages
+// its K block (32 x D) and V^T block (D x 32) in LDS of its own by direct
+// global -> LDS DMA, whole rows at a time (fragments read straight from global
+// memory touch 32 lines per instruction: 30 us for 438 + 300 tokens against
+// 25; 23 tokens 8.0 us).  The next block's K is requested when this one's
+// fragments are in registers, its V^T when this one's products are done.  What
+// bounds it is the chain of one wave's key blocks (up to 4 here): the
+// accumulators, q and K take the registers of one wave per SIMD, so nothing
+// hides a block's LDS reads and exponentials.
+// S^T = K Q^T (K rows as the first MFMA operand, q in registers), so a lane
+// holds 16 keys of one query, exactly what it feeds back as the P^T operand of
+// O^T = V^T P^T: the contraction takes key 16 s + 8 (e / 4) + 4 (lane / 32) + e %
+// 4 as element e of step s, the order in which gemma_qkv_kernel stores V^T
+// within each 16 keys, so nothing crosses lanes.
+// LDS rows: 16-byte chunk c of K row r at slot c ^ (r & 15) (D 64: c ^ ((r >> 1)
+// & 7)), of V^T row r at c ^ ((r >> 2) & 3): 16 consecutive rows at one chunk meet
+// 16 distinct bank groups.
+template <int D>
+__global__ __launch_bounds__(256, 1) void gemma_attention_kernel(const f16 * __restrict__ q16,
+                                                                 const f16 * __restrict__ k16,
+                                                                 const f16 * __restrict__ vt16, GemmaSeqs sq,
+                                                                 int nh, int nkv, float cap, int window,
+                                                                 f16 * __restrict__ o16) {
+    const float inv_cap = 1.0f / cap;
+    constexpr int KS = D / 16, DT = D / 32;  // 16-deep steps over d, 32-row tiles of O^T
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    float4 * part = reinterpret_cast<float4 *>(lds);                      // [wave][DT][4][64]
+    float * stat = reinterpret_cast<float *>(lds + 4 * DT * 4 * 64 * 16);  // [wave][max, sum][32]
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int ql = lane & 31, hf = lane >> 5;
+    const int h = blockIdx.y, kvh = h / (nh / nkv);
+    const int nb0 = (sq.T[0] + 31) / 32;
+    const int si = (int)blockIdx.x >= nb0 ? 1 : 0;
+    // the longest rows first
+    const int nb = (sq.T[si] + 31) / 32, qb = nb - 1 - ((int)blockIdx.x - (si ? nb0 : 0));
+    const int T = sq.T[si], Tp = sq.Tp[si];
+    const int64_t row0 = sq.row0[si];
+    const int q0 = qb * 32, tq = min(q0 + ql, T - 1);
+    const f16 * qr = q16 + ((row0 + tq) * nh + h) * D + 8 * hf;
+    f16x8 qf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const f16x8 *>(qr + 16 * s);
+    const f16 * vb = vt16 + sq.vt_off[si] + (int64_t)kvh * D * Tp;
+    const f16 * kbase = k16 + (row0 * nkv + kvh) * D;
+    const int kb_first = window > 0 ? max(0, q0 - window + 1) / 32 : 0, kb_last = min(q0 + 31, T - 1) / 32;
+    constexpr int CPR = D / 8;  // 16-byte chunks of a K row
+    unsigned char * kl = lds + w * (2 * D * 64), * vl = kl + D * 64;
+    auto ksw = [](int r) { return D == 64 ? (r >> 1) & 7 : r & 15; };
+    // (blocks past the last: the last again, never used)
+    auto load_k = [&](int kb) {
+        const int k0 = min(kb, kb_last) * 32;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const int n = i * 64 + lane, r = n / CPR, c = (n % CPR) ^ ksw(r);
+            __builtin_amdgcn_global_load_lds(
+                static_cast<const void *>(kbase + ((unsigned)min(k0 + r, T - 1) * (unsigned)(nkv * D) + c * 8)),
+                SANA_LDS(kl + i * 1024), 16, 0, 0);
+        }
+    };
+    auto load_v = [&](int kb) {
+        const int k0 = min(kb, kb_last) * 32;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const int n = i * 64 + lane, r = n / 4, c = (n % 4) ^ ((r >> 2) & 3);
+            __builtin_amdgcn_global_load_lds(static_cast<const void *>(vb + ((unsigned)(r * Tp) + k0 + c * 8)),
+                                             SANA_LDS(vl + i * 1024), 16, 0, 0);
+        }
+    };
+    load_k(kb_first + w);
+    load_v(kb_first + w);
+    f32x16 o[DT];
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[j][e] = 0.0f;
+    float mx = -INFINITY, sum = 0.0f;
+    for (int kb = kb_first + w; kb <= kb_last; kb += 4) {
+        const int k0 = kb * 32;
+        f16x8 kf[KS];
+        wait_vmcnt<KS>();  // K has landed, V^T may be in flight
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            kf[s] = *reinterpret_cast<const f16x8 *>(kl + ql * (D * 2) + (((2 * s + hf) ^ ksw(ql)) << 4));
+        wait_lgkmcnt0();
+        load_k(kb + 4);
+        f32x16 sc, sd;  // even and odd steps: two MFMA chains
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[e] = sd[e] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; s += 2) {
+            sc = mfma_32x32x16(kf[s], qf[s], sc);
+            sd = mfma_32x32x16(kf[s + 1], qf[s + 1], sd);
+        }
+        // lane: query q0 + ql, keys k0 + 8 (e / 4) + 4 hf + e % 4
+        float bm = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int j = k0 + 8 * (e >> 2) + 4 * hf + (e & 3), t = q0 + ql;
+            const bool in = j <= t && j < T && (window <= 0 || j > t - window);
+            sc[e] = in ? cap * tanh_f32((sc[e] + sd[e]) * inv_cap) : -INFINITY;
+            bm = fmaxf(bm, sc[e]);
+        }
+        bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+        const float mn = fmaxf(mx, bm);
+        // a query without a key so far keeps sums of zero
+        const float f = mx == -INFINITY ? 0.0f : exp_f32(mx - mn);
+        float bs = 0.0f;
+        f16x8 pf[2];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const float p = sc[e] == -INFINITY ? 0.0f : exp_f32(sc[e] - mn);
+            bs += p;
+            pf[e >> 3][e & 7] = (f16)p;
+        }
+        bs += __shfl_xor(bs, 32, 64);
+        sum = sum * f + bs;
+        mx = mn;
+        if (!__all(f == 1.0f)) {  // a new maximum somewhere
+#pragma unroll
+            for (int j = 0; j < DT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[j][e] *= f;
+        }
+        wait_vmcnt<KS>();  // V^T has landed, the next K may be in flight
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int j = 0; j < DT; ++j) {
+                const int r = j * 32 + ql;
+                const f16x8 v =
+                    *reinterpret_cast<const f16x8 *>(vl + r * 64 + (((2 * s + hf) ^ ((r >> 2) & 3)) << 4));
+                o[j] = mfma_32x32x16(v, pf[s], o[j]);
+            }
+        wait_lgkmcnt0();
+        load_v(kb + 4);
+    }
+    wait_vmcnt<0>();
+    const int64_t qrow = ((row0 + q0 + ql) * nh + h) * (int64_t)D;
+    auto store4 = [&](int i, const float4 & a, float rs) {  // 4 consecutive d: 32 (i / 4) + 8 (i % 4) + 4 hf
+        f16x4 hv;
+        hv[0] = (f16)(a.x * rs);
+        hv[1] = (f16)(a.y * rs);
+        hv[2] = (f16)(a.z * rs);
+        hv[3] = (f16)(a.w * rs);
+        *reinterpret_cast<f16x4 *>(o16 + qrow + 32 * (i >> 2) + 8 * (i & 3) + 4 * hf) = hv;
+    };
+    // waves that had keys; alone, the first one stores
+    const int nw = min(4, kb_last - kb_first + 1);
+    if (nw == 1) {
+        if (w > 0 || q0 + ql >= T) return;
+        const float rs = 1.0f / sum;
+#pragma unroll
+        for (int i = 0; i < DT * 4; ++i) {
+            const f32x16 & t = o[i >> 2];
+            store4(i, make_float4(t[4 * (i & 3)], t[4 * (i & 3) + 1], t[4 * (i & 3) + 2], t[4 * (i & 3) + 3]), rs);
+        }
+        return;
+    }
+    // merge the waves: common max, scaled sums and outputs
+    if (hf == 0) {
+        stat[w * 64 + ql] = mx;
+        stat[w * 64 + 32 + ql] = sum;
+    }
+    __syncthreads();  // also: every wave is done with its K and V^T
+    float gm = -INFINITY, gs = 0.0f;
+    for (int v = 0; v < nw; ++v) gm = fmaxf(gm, stat[v * 64 + ql]);
+    for (int v = 0; v < nw; ++v) {
+        const float m = stat[v * 64 + ql];
+        gs += m == -INFINITY ? 0.0f : stat[v * 64 + 32 + ql] * exp_f32(m - gm);
+    }
+    if (w < nw) {
+        const float f = mx == -INFINITY ? 0.0f : exp_f32(mx - gm);
+#pragma unroll
+        for (int j = 0; j < DT; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                part[((w * DT + j) * 4 + q) * 64 + lane] =
+                    make_float4(o[j][4 * q] * f, o[j][4 * q + 1] * f, o[j][4 * q + 2] * f, o[j][4 * q + 3] * f);
+    }
+    __syncthreads();
+    if (q0 + ql >= T) return;
+    const float rs = 1.0f / gs;
+    for (int i = w; i < DT * 4; i += 4) {
+        float4 a = part[i * 64 + lane];
+        for (int v = 1; v < nw; ++v) {
+            const float4 b = part[(v * DT * 4 + i) * 64 + lane];
+            a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+        }
+        store4(i, a, rs);
+    }
+}
+
+template <int D>
+hipError_t launch_gemma_attention(const f16 * q, const f16 * k, const f16 * vt, const GemmaSeqs & sq, int nh, int nkv,
+                                  float cap, int window, f16 * o, hipStream_t s) {
+    constexpr int lds = 4 * (D / 32) * 4 * 64 * 16 + 4 * 64 * 4;
+    static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemma_attention_kernel<D>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+    (void)ok;
+    int blocks = 0;
+    for (int i = 0; i < sq.n; ++i) blocks += (sq.T[i] + 31) / 32;
+    hipLaunchKernelGGL((gemma_attention_kernel<D>), dim3((unsigned)blocks, (unsigned)nh), dim3(256), lds, s, q, k, vt,
+                       sq, nh, nkv, cap, window, o);
+    return hipGetLastError();
 }
 
 // Rows (head, t) of S [nh][T][Tp]: s = cap * tanh(S / cap) over keys j <= t
@@ -225,11 +527,6 @@ struct sana_gemma {
     std::map<std::string, bool> loaded;
     std::vector<std::string> required;
     hipStream_t stream = nullptr;
-    // second stream: the attention of every other sequence runs on it, beside
-    // the first sequence's (fork after the q|k|v projection, join before the
-    // output projection of each layer)
-    hipStream_t stream2 = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     // workspace: rows of all sequences of one encode, and the per-sequence
     // attention buffers (V^T, scores, probabilities) back to back
     int64_t ws_M = 0, ws_vt = 0, ws_att = 0;
@@ -239,9 +536,6 @@ struct sana_gemma {
     std::map<std::vector<int64_t>, hipGraphExec_t> graphs;
     ~sana_gemma() {
         for (auto & kv : graphs) (void)hipGraphExecDestroy(kv.second);
-        if (ev_fork) (void)hipEventDestroy(ev_fork);
-        if (ev_join) (void)hipEventDestroy(ev_join);
-        if (stream2) (void)hipStreamDestroy(stream2);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -380,6 +674,11 @@ std::vector<Seq> layout(const sana_gemma * g, const std::vector<int64_t> & lens)
     return q;
 }
 
+bool one_pass_attention(const sana_gemma_config & c) {
+    // (32-bit offsets into the K rows: up to 8192 tokens)
+    return (c.head_dim == 64 || c.head_dim == 128 || c.head_dim == 256) && c.kv_heads * c.head_dim <= 65536;
+}
+
 void ensure_workspace(sana_gemma * g, const std::vector<Seq> & q) {
     const Seq & e = q.back();
     const int64_t M = e.row0 + e.T, vt = e.vt_off + g->Dkv * e.Tp, att = e.att_off + g->cfg.heads * e.T * e.Tp;
@@ -399,8 +698,10 @@ void ensure_workspace(sana_gemma * g, const std::vector<Seq> & q) {
     g->q16.ensure(R * g->Dq * 2, false);
     g->k16.ensure(R * g->Dkv * 2, false);
     g->vt16.ensure((size_t)g->ws_vt * 2, false);
-    g->s32.ensure((size_t)g->ws_att * 4, false);
-    g->p16.ensure((size_t)g->ws_att * 2, false);
+    if (!one_pass_attention(c)) {
+        g->s32.ensure((size_t)g->ws_att * 4, false);
+        g->p16.ensure((size_t)g->ws_att * 2, false);
+    }
     g->o16.ensure(R * g->Dq * 2, false);
     g->g16.ensure(R * c.ffn * 2, false);
     g->out32.ensure(R * H * 4, false);
@@ -456,22 +757,29 @@ void gemm_batched(const half_t * A, int64_t lda, int64_t sa, const half_t * W, i
     launch_check(sana::gemm(p, s), "gemma batched gemm");
 }
 
-void norm(const sana_gemma * g, const float * y, int64_t M, const DevMem & w, int mode, half_t * o16, float * o32,
-          hipStream_t s, int parts = 1, const DevMem * w2 = nullptr) {
-    const int64_t C = g->cfg.hidden;
+template <int MODE, int PARTS>
+void norm_as(const float * y, int64_t M, int64_t C, const float * w, float eps, f16 * o16, float * o32,
+             const float * w2, hipStream_t s) {
     const dim3 grid((unsigned)M), blk(256);
-    f16 * h = reinterpret_cast<f16 *>(o16);
-    const float eps = g->cfg.rms_eps;
-    const int64_t pstride = M * C;
-    const float * w2p = w2 ? w2->as<float>() : nullptr;
-#define SANA_GEMMA_NORM(n4)                                                                                      \
-    hipLaunchKernelGGL((gemma_norm_kernel<n4>), grid, blk, 0, s, y, parts, pstride, (int)C, (int)M, w.as<float>(), \
-                       eps, mode, h, o32, w2p)
+#define SANA_GEMMA_NORM(n4) \
+    hipLaunchKernelGGL((gemma_norm_kernel<n4, MODE, PARTS>), grid, blk, 0, s, y, M * C, (int)C, w, eps, o16, o32, w2)
     if (C <= 1024) SANA_GEMMA_NORM(1);
     else if (C <= 2048) SANA_GEMMA_NORM(2);
+    else if (C <= 3072) SANA_GEMMA_NORM(3);
     else SANA_GEMMA_NORM(4);
 #undef SANA_GEMMA_NORM
     launch_check(hipGetLastError(), "gemma norm");
+}
+
+template <int MODE>
+void norm(const sana_gemma * g, const float * y, int64_t M, const DevMem & w, half_t * o16, float * o32,
+          hipStream_t s, int parts = 1, const DevMem * w2 = nullptr) {
+    const int64_t C = g->cfg.hidden;
+    f16 * h = reinterpret_cast<f16 *>(o16);
+    const float * w2p = w2 ? w2->as<float>() : nullptr;
+    if (parts == 1) norm_as<MODE, 1>(y, M, C, w.as<float>(), g->cfg.rms_eps, h, o32, w2p, s);
+    else if (parts == 2) norm_as<MODE, 2>(y, M, C, w.as<float>(), g->cfg.rms_eps, h, o32, w2p, s);
+    else norm_as<MODE, 4>(y, M, C, w.as<float>(), g->cfg.rms_eps, h, o32, w2p, s);
 }
 
 // Split-K factor of an M x H output with contraction K: the down and output
@@ -492,6 +800,38 @@ int split_k(int64_t K) {
 // K / 64 tile latencies.  Depends on K only, as split_k.
 int k_runs(int64_t K) { return K >= 1024 ? 4 : 1; }
 
+// Attention of other head dims: per sequence the scores of all heads as one
+// batched product (head h uses K head h / grp), the softmax, and the batched
+// P.V product.
+void attention_by_products(sana_gemma * g, const std::vector<Seq> & seqs, int window, hipStream_t s) {
+    const sana_gemma_config & c = g->cfg;
+    const int64_t d = c.head_dim, nh = c.heads, Dq = g->Dq, Dkv = g->Dkv, grp = nh / c.kv_heads;
+    for (const Seq & q : seqs) {
+        const int64_t T = q.T, Tp = q.Tp;
+        const half_t * q16 = g->q16.as<half_t>() + q.row0 * Dq;
+        const half_t * k16 = g->k16.as<half_t>() + q.row0 * Dkv;
+        const half_t * vt16 = g->vt16.as<half_t>() + q.vt_off;
+        float * s32 = g->s32.as<float>() + q.att_off;
+        half_t * p16 = g->p16.as<half_t>() + q.att_off;
+        gemm_batched(q16, Dq, d, k16, Dkv, d, (int)grp, T, T, d, nullptr, 0, 0, s32, Tp, T * Tp, (int)nh, s);
+        const dim3 sg((unsigned)((nh * T + 3) / 4)), sb(256);
+        f16 * pp = reinterpret_cast<f16 *>(p16);
+#define SANA_GEMMA_SOFTMAX(nj)                                                                                \
+    hipLaunchKernelGGL((gemma_softmax_kernel<nj>), sg, sb, 0, s, s32, pp, (int)nh, (int)T, (int)Tp, c.attn_softcap, \
+                       window)
+        // Tp <= 64 NJ (token counts up to 8192: Tp <= 8192)
+        if (Tp <= 512) SANA_GEMMA_SOFTMAX(8);
+        else if (Tp <= 1024) SANA_GEMMA_SOFTMAX(16);
+        else if (Tp <= 2048) SANA_GEMMA_SOFTMAX(32);
+        else if (Tp <= 4096) SANA_GEMMA_SOFTMAX(64);
+        else SANA_GEMMA_SOFTMAX(128);
+#undef SANA_GEMMA_SOFTMAX
+        launch_check(hipGetLastError(), "gemma softmax");
+        gemm_batched(p16, Tp, T * Tp, vt16, Tp, d * Tp, (int)grp, T, d, Tp, g->o16.as<half_t>() + q.row0 * Dq, Dq, d,
+                     nullptr, 0, 0, (int)nh, s);
+    }
+}
+
 // decode_embeddings (src/gemma_encoder.cpp:95-152) on device token ids, for
 // one or more independent sequences at once: their rows share every
 // per-token kernel (norms, the projections, GeGLU) and only the attention
@@ -501,7 +841,7 @@ int k_runs(int64_t K) { return K >= 1024 ? 4 : 1; }
 void encode(sana_gemma * g, const std::vector<Seq> & seqs, hipStream_t s) {
     const sana_gemma_config & c = g->cfg;
     const int64_t H = c.hidden, F = c.ffn, d = c.head_dim, nh = c.heads, nkv = c.kv_heads;
-    const int64_t Dq = g->Dq, Dkv = g->Dkv, Dqkv = Dq + 2 * Dkv, grp = nh / nkv;
+    const int64_t Dq = g->Dq, Dkv = g->Dkv, Dqkv = Dq + 2 * Dkv;
     const int64_t M = seqs.back().row0 + seqs.back().T;
     hipLaunchKernelGGL(gemma_embed_kernel, dim3(blocks_for(M * H)), dim3(256), 0, s, g->tok.as<int32_t>(),
                        g->emb16.as<f16>(), g->x32.as<float>(), (int)M, (int)H, std::sqrt((float)H));
@@ -511,72 +851,52 @@ void encode(sana_gemma * g, const std::vector<Seq> & seqs, hipStream_t s) {
         LayerDev & L = *g->layers[l];
         // the pre-attention norm: layer 0 here, later layers in the previous
         // layer's last norm launch
-        if (l == 0) norm(g, g->x32.as<float>(), M, L.n_attn, 0, a16, nullptr, s);
+        if (l == 0) norm<0>(g, g->x32.as<float>(), M, L.n_attn, a16, nullptr, s);
         gemm(a16, H, L.wqkv.as<half_t>(), H, M, Dqkv, H, nullptr, 0, g->qkv32.as<float>(), Dqkv, s, sana::kActNone,
              k_runs(H));
         const int window = (c.sliding_window > 0 && l % 2 == 0) ? (int)c.sliding_window : 0;
-        // sequences 1, 3, ... on the second stream (their buffers are disjoint)
-        const bool two = seqs.size() > 1;
-        if (two) {
-            hip_check(hipEventRecord(g->ev_fork, s), "hipEventRecord");
-            hip_check(hipStreamWaitEvent(g->stream2, g->ev_fork, 0), "hipStreamWaitEvent");
+        GemmaSeqs sq{};
+        sq.n = (int)seqs.size();
+        int vblocks = 0;
+        for (int i = 0; i < sq.n; ++i) {
+            sq.row0[i] = (int)seqs[i].row0;
+            sq.T[i] = (int)seqs[i].T;
+            sq.Tp[i] = (int)seqs[i].Tp;
+            sq.vt_off[i] = seqs[i].vt_off;
+            vblocks += (int)(seqs[i].Tp / 64 * (nkv * d / 64));
         }
-        for (size_t si = 0; si < seqs.size(); ++si) {
-            const Seq & q = seqs[si];
-            const hipStream_t ss = (si & 1) ? g->stream2 : s;
-            const int64_t T = q.T, Tp = q.Tp;
-            half_t * q16 = g->q16.as<half_t>() + q.row0 * Dq;
-            half_t * k16 = g->k16.as<half_t>() + q.row0 * Dkv;
-            half_t * vt16 = g->vt16.as<half_t>() + q.vt_off;
-            float * s32 = g->s32.as<float>() + q.att_off;
-            half_t * p16 = g->p16.as<half_t>() + q.att_off;
-            const int64_t n = T * (nh + nkv) * (d / 2) + nkv * d * Tp;
-            hipLaunchKernelGGL(gemma_qkv_kernel, dim3(blocks_for(n)), dim3(256), 0, ss,
-                               g->qkv32.as<float>() + q.row0 * Dqkv, (int)T, (int)Tp, (int)nh, (int)nkv, (int)d,
-                               c.rope_theta, c.query_scale, reinterpret_cast<f16 *>(q16),
-                               reinterpret_cast<f16 *>(k16), reinterpret_cast<f16 *>(vt16));
-            launch_check(hipGetLastError(), "gemma qkv");
-            // scores of all heads in one launch: head h uses K head h / grp
-            gemm_batched(q16, Dq, d, k16, Dkv, d, (int)grp, T, T, d, nullptr, 0, 0, s32, Tp, T * Tp, (int)nh, ss);
-            {
-                const dim3 sg((unsigned)((nh * T + 3) / 4)), sb(256);
-                f16 * pp = reinterpret_cast<f16 *>(p16);
-#define SANA_GEMMA_SOFTMAX(nj)                                                                                 \
-    hipLaunchKernelGGL((gemma_softmax_kernel<nj>), sg, sb, 0, ss, s32, pp, (int)nh, (int)T, (int)Tp, c.attn_softcap, \
-                       window)
-                // Tp <= 64 NJ (token counts up to 8192: Tp <= 8192)
-                if (Tp <= 512) SANA_GEMMA_SOFTMAX(8);
-                else if (Tp <= 1024) SANA_GEMMA_SOFTMAX(16);
-                else if (Tp <= 2048) SANA_GEMMA_SOFTMAX(32);
-                else if (Tp <= 4096) SANA_GEMMA_SOFTMAX(64);
-                else SANA_GEMMA_SOFTMAX(128);
-#undef SANA_GEMMA_SOFTMAX
-                launch_check(hipGetLastError(), "gemma softmax");
-            }
-            gemm_batched(p16, Tp, T * Tp, vt16, Tp, d * Tp, (int)grp, T, d, Tp, g->o16.as<half_t>() + q.row0 * Dq,
-                         Dq, d, nullptr, 0, 0, (int)nh, ss);
-        }
-        if (two) {
-            hip_check(hipEventRecord(g->ev_join, g->stream2), "hipEventRecord");
-            hip_check(hipStreamWaitEvent(s, g->ev_join, 0), "hipStreamWaitEvent");
-        }
+        const int rblocks = (int)blocks_for(M * ((nh + nkv + 3) / 4) * (d / 2));
+        f16 * q16 = g->q16.as<f16>();
+        f16 * k16 = g->k16.as<f16>();
+        f16 * vt16 = g->vt16.as<f16>();
+        f16 * o16 = g->o16.as<f16>();
+        hipLaunchKernelGGL(gemma_qkv_kernel, dim3((unsigned)(rblocks + vblocks)), dim3(256), 0, s,
+                           g->qkv32.as<float>(), sq, (int)M, (int)nh, (int)nkv, (int)d, c.rope_theta, c.query_scale,
+                           rblocks, one_pass_attention(c) ? 1 : 0, q16, k16, vt16);
+        launch_check(hipGetLastError(), "gemma qkv");
+        hipError_t ae = hipSuccess;
+        if (!one_pass_attention(c)) attention_by_products(g, seqs, window, s);
+        else if (d == 64) ae = launch_gemma_attention<64>(q16, k16, vt16, sq, (int)nh, (int)nkv, c.attn_softcap, window, o16, s);
+        else if (d == 128) ae = launch_gemma_attention<128>(q16, k16, vt16, sq, (int)nh, (int)nkv, c.attn_softcap, window, o16, s);
+        else ae = launch_gemma_attention<256>(q16, k16, vt16, sq, (int)nh, (int)nkv, c.attn_softcap, window, o16, s);
+        launch_check(ae, "gemma attention");
         const int so = split_k(Dq);
         gemm_batched(g->o16.as<half_t>(), Dq, Dq / so, L.wo.as<half_t>(), Dq, Dq / so, 1, M, H, Dq / so, nullptr, 0,
                      0, g->y32.as<float>(), H, M * H, so, s, k_runs(Dq / so));
         // x += post-attention norm of the projection, then the pre-FFN norm
-        norm(g, g->y32.as<float>(), M, L.n_post_attn, 3, a16, g->x32.as<float>(), s, so, &L.n_ffn);
+        norm<3>(g, g->y32.as<float>(), M, L.n_post_attn, a16, g->x32.as<float>(), s, so, &L.n_ffn);
         gemm(a16, H, L.wgu.as<half_t>(), H, M, 2 * F, H, g->g16.as<half_t>(), F, nullptr, 0, s, sana::kActGeglu);
         const int sd = split_k(F);
         gemm_batched(g->g16.as<half_t>(), F, F / sd, L.wdown.as<half_t>(), F, F / sd, 1, M, H, F / sd, nullptr, 0, 0,
                      g->y32.as<float>(), H, M * H, sd, s, k_runs(F / sd));
         // x += post-FFN norm, then the next layer's pre-attention norm
         if (l + 1 < c.layers)
-            norm(g, g->y32.as<float>(), M, L.n_post_ffw, 3, a16, g->x32.as<float>(), s, sd,
-                 &g->layers[l + 1]->n_attn);
+            norm<3>(g, g->y32.as<float>(), M, L.n_post_ffw, a16, g->x32.as<float>(), s, sd,
+                    &g->layers[l + 1]->n_attn);
         else
-            norm(g, g->y32.as<float>(), M, L.n_post_ffw, 1, nullptr, g->x32.as<float>(), s, sd);
+            norm<1>(g, g->y32.as<float>(), M, L.n_post_ffw, nullptr, g->x32.as<float>(), s, sd);
     }
-    norm(g, g->x32.as<float>(), M, g->out_norm, 2, nullptr, g->out32.as<float>(), s);
+    norm<2>(g, g->x32.as<float>(), M, g->out_norm, nullptr, g->out32.as<float>(), s);
 }
 
 // Encodes the token sequences seqs[i] (host ids, lengths lens[i]) into
@@ -662,9 +982,6 @@ int sana_gemma_create(const sana_gemma_config * cfg, sana_gemma ** out) {
         for (int64_t l = 0; l < cfg->layers; ++l) g->layers.push_back(std::make_unique<LayerDev>());
         g->required = required_names(g.get());
         hip_check(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking), "hipStreamCreate");
-        hip_check(hipStreamCreateWithFlags(&g->stream2, hipStreamNonBlocking), "hipStreamCreate");
-        hip_check(hipEventCreateWithFlags(&g->ev_fork, hipEventDisableTiming), "hipEventCreate");
-        hip_check(hipEventCreateWithFlags(&g->ev_join, hipEventDisableTiming), "hipEventCreate");
         *out = g.release();
     });
 }

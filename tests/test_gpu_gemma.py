@@ -159,3 +159,38 @@ def test_rejects_bad_input():
         assert e.value.code == sana_dit.SANA_ERR_SHAPE
     finally:
         dev.close()
+
+
+EDGE = dict(vocab=50, hidden=192, layers=2, heads=4, kv_heads=2, head_dim=64, ffn=128, sliding_window=0, rms_eps=1e-6,
+            rope_theta=10000.0, softcap=50.0, query_scale=1 / 8)
+
+
+@pytest.mark.parametrize("d", [64, 128, 192, 256])
+@pytest.mark.parametrize("T,window", [(1, 0), (31, 0), (32, 5), (33, 40), (65, 64), (97, 33), (130, 1), (161, 0),
+                                      (300, 100)])
+def test_attention_edges_vs_oracle(d, T, window):
+    """Query and key blocks of 32, windows that start inside, at and outside a
+    block, single rows; head dim 192 takes the product path."""
+    cfg = dict(EDGE, head_dim=d, sliding_window=window, query_scale=d ** -0.5)
+    w, dev = build(cfg, scale=0.1)
+    try:
+        tokens = np.random.default_rng(T + d).integers(0, cfg["vocab"], size=T)
+        got = dev.encode(tokens)
+        assert rel_l2(got, G.forward(w, cfg, tokens)) < TOL
+        other = np.random.default_rng(T).integers(0, cfg["vocab"], size=max(1, T // 2))
+        a, b = dev.encode_pair(other, tokens)
+        assert np.array_equal(b, got) and np.array_equal(a, dev.encode(other))
+    finally:
+        dev.close()
+
+
+@pytest.mark.parametrize("hidden,ffn", [(64, 64), (1088, 128), (2112, 8192), (3136, 64), (4096, 64)])
+def test_norm_widths_vs_oracle(hidden, ffn):
+    """Row widths of one to four 1024-channel runs, one, two and four split-K partials."""
+    cfg = dict(EDGE, hidden=hidden, ffn=ffn, heads=16 if ffn > 64 else 4)
+    w, dev = build(cfg, scale=0.03)
+    try:
+        tokens = np.random.default_rng(hidden).integers(0, cfg["vocab"], size=21)
+        assert rel_l2(dev.encode(tokens), G.forward(w, cfg, tokens)) < TOL
+    finally:
+        dev.close()
