@@ -13,7 +13,9 @@
 //     stage is refilled with tile kt+STAGES, so each load has STAGES-1 tiles
 //     of MFMA work to land.  Completion is tracked with an explicit vmcnt
 //     wait (the loads of later tiles stay outstanding) and one s_barrier per
-//     k-tile, placed after the tile's last MFMAs are issued.
+//     k-tile, placed after the tile's last MFMAs are issued (schedule 2: before
+//     the last quarter of them, which then covers the barrier and the next
+//     tile's first LDS reads).
 //   * LDS rows are 128 bytes; 16-byte chunk c of row r is stored in slot
 //     c ^ ((r >> 1) & 7).  The DMA writes lane l to slot l & 7 of row l >> 3 of
 //     its 8-row block, so lane l fetches the chunk that maps there.  gfx950's
@@ -87,7 +89,9 @@ struct Cfg {
     static constexpr int EPI_ROWS =
         (BM * (BN + CPAD) * 4 <= (RING_BYTES > 80 * 1024 ? RING_BYTES : 80 * 1024)) ? BM : WTM;
     static constexpr int EPI_BYTES = EPI_ROWS * (BN + CPAD) * 4;
-    static constexpr int LDS_BYTES = (RING_BYTES > EPI_BYTES) ? RING_BYTES : EPI_BYTES;
+    static constexpr int EPI16_BYTES = BM * (BN + 8) * 2;  // the fp16 epilogue's tile, always whole
+    static constexpr int EPI_MAX = EPI_BYTES > EPI16_BYTES ? EPI_BYTES : EPI16_BYTES;
+    static constexpr int LDS_BYTES = RING_BYTES > EPI_MAX ? RING_BYTES : EPI_MAX;
     static constexpr int PART_BYTES = GW * TM * TN * 4096;  // one k-group's sums
     static_assert((KG - 1) * PART_BYTES <= LDS_BYTES, "k-group partial sums");
     static_assert(BM % (8 * GW) == 0 && BN % (8 * GW) == 0, "tile rows must split into 8-row wave loads");
@@ -113,7 +117,7 @@ template <int BM, int BN, int WM, int WN, int STAGES, int MODE, int SCHED, int A
           int SEG = 1>
 __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in) {
     using G = Cfg<BM, BN, WM, WN, STAGES, KG>;
-    static_assert((KG == 1 || SCHED == 1) && (SEG == 1 || (KG == 1 && SCHED != 0 && SCHED != 2)), "schedule");
+    static_assert((KG == 1 || SCHED == 1) && (SEG == 1 || (KG == 1 && SCHED != 2)), "schedule");
     // product blockIdx.y of a batched launch (plain stores only)
     GemmParams p = p_in;
     if constexpr (MODE == kGemmStore && CONV == 0) {
@@ -231,10 +235,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in
     const int brow0 = wn * G::WTN + (lane & 31);
     const int khalf = lane >> 5;
 
-    // Operand fragments are double-buffered in registers: the LDS reads of
-    // k-step s+1 are in flight while the MFMAs of step s run.  The tile
-    // boundary (wait for the next tile's DMA, barrier, refill the freed stage)
-    // is placed after the last step's MFMAs are issued, so it overlaps them.
+    // Fragments of a whole k-tile (schedules 1 and 3) or of two MFMA k-steps (2).
     constexpr int NS = kBK / 16;               // MFMA k-steps per tile
     constexpr int NB = (SCHED == 1 || SCHED == 3) ? NS : 2;    // fragment buffers
     f16x8 af[NB][G::TM], bf[NB][G::TN];
@@ -422,10 +423,13 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in
             }
         }
     } else {
-        // Operand fragments double-buffered in registers: the LDS reads of
-        // k-step s+1 are in flight while the MFMAs of step s run.  The tile
-        // boundary (wait for the next tile's DMA, barrier, refill the freed
-        // stage) follows the last step's MFMAs, so it overlaps them.
+        // Operand fragments double-buffered in registers: the LDS reads of k-step
+        // s+1 go out between the MFMAs of step s.  The tile boundary (wait for the
+        // next tile's DMA, barrier, refill of the freed stage) comes before the last
+        // step's MFMAs, whose fragments are in registers by then, and the next tile's
+        // first fragments are requested there too: those MFMAs cover the barrier and
+        // the reads, so one workgroup per CU can keep the matrix cores busy.
+        constexpr int RD = G::TM + G::TN, MF = G::TM * G::TN;
         load_frags(0, 0, 0);
         for (int kt = 0; kt < NT_K; ++kt) {
             const int st = kt % STAGES;
@@ -433,22 +437,24 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in
             for (int s = 0; s < NS - 1; ++s) {
                 load_frags(st, s + 1, (s + 1) & 1);
                 mfmas(s & 1);
-                if constexpr (SCHED == 2) {
-                    __builtin_amdgcn_sched_group_barrier(0x100, G::TM + G::TN, 0);  // DS reads of step s+1
-                    __builtin_amdgcn_sched_group_barrier(0x008, G::TM * G::TN, 0);  // then MFMAs of step s
+#pragma unroll
+                for (int q = 0; q < RD; ++q) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                   // an LDS read of step s+1
+                    __builtin_amdgcn_sched_group_barrier(0x008, (MF + RD - 1) / RD, 0);  // MFMAs of step s
                 }
-            }
-            mfmas((NS - 1) & 1);
-            if (kt + 1 < NT_K) {
                 __builtin_amdgcn_sched_barrier(0);
-                // tile kt+1 has landed (this wave's DMA), then every wave's has and
-                // every wave is done reading stage st, which takes tile kt+STAGES.
+            }
+            if (kt + 1 < NT_K) {
+                // this wave's reads of stage st have returned and its part of tile kt+1
+                // has landed; after the barrier every wave's
+                wait_lgkmcnt0();
                 wait_stages<G::LOADS, STAGES>(min(STAGES - 2, NT_K - 2 - kt));
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_sched_barrier(0);
-                if (kt + STAGES < NT_K) issue(kt + STAGES, st);
                 load_frags((kt + 1) % STAGES, 0, 0);
+                if (kt + STAGES < NT_K) issue(kt + STAGES, st);
             }
+            mfmas((NS - 1) & 1);
         }
     }
 
@@ -960,7 +966,17 @@ hipError_t launch_conv_kg(const GemmParams & p, hipStream_t s) {
     return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActNone, CONV, KG>(p, tiles, s);
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, int SCHED = 0>
+// 256 x 256 tiles (8 waves of 128 x 64, one workgroup per CU): stores and the q|k|v split.
+hipError_t launch256(const GemmParams & p, hipStream_t s) {
+    const int tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
+    if (p.mode == kGemmQKV) return launch_mode<256, 256, 2, 4, 2, kGemmQKV, 2, kActNone>(p, tiles, s);
+    if (p.act == kActSilu) return launch_mode<256, 256, 2, 4, 2, kGemmStore, 2, kActSilu>(p, tiles, s);
+    if (p.act == kActGelu) return launch_mode<256, 256, 2, 4, 2, kGemmStore, 2, kActGelu>(p, tiles, s);
+    if (p.act == kActGeglu) return launch_mode<256, 256, 2, 4, 2, kGemmStore, 2, kActGeglu>(p, tiles, s);
+    return launch_mode<256, 256, 2, 4, 2, kGemmStore, 2, kActNone>(p, tiles, s);
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES, int SCHED>
 hipError_t launch(const GemmParams & p, hipStream_t s) {
     const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
     if (p.mode == kGemmResidual) return launch_mode<BM, BN, WM, WN, STAGES, kGemmResidual, SCHED, kActNone>(p, tiles, s);
@@ -1027,17 +1043,27 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     // tiles of the rows that decide the order of the k sums
     const int64_t rows = p.order_rows > 0 ? p.order_rows : p.M;
     auto grid = [&](int bm, int bn) { return (rows + bm - 1) / bm * ((p.N + bn - 1) / bn) * co; };
+    // Rounds (in 1/64) of `slots` workgroups at a time that bm x bn tiles of all
+    // rows take; launches that share the CUs fill each other's last round.
+    auto rounds = [&](int bm, int bn, int64_t slots) {
+        const int64_t t = ((int64_t)p.M + bm - 1) / bm * ((p.N + bn - 1) / bn) * co;
+        return co > 1 ? std::max<int64_t>(64, t * 64 / slots) : (t + slots - 1) / slots * 64;
+    };
     if (p.conv) {
         if (grid(32, 64) <= 288)
             return p.conv == 2 ? launch_conv_kg<32, 64, 1, 2, 3, 2, 4>(p, s) : launch_conv_kg<32, 64, 1, 2, 3, 1, 4>(p, s);
         if (grid(64, 64) <= 320)
             return p.conv == 2 ? launch_conv_kg<64, 64, 2, 2, 4, 2, 2>(p, s) : launch_conv_kg<64, 64, 2, 2, 4, 1, 2>(p, s);
-        // Early stage release is 2-6 % faster than schedule 1 on the VAE's
-        // 3x3 convs (1024^2 x 128, 512^2 x 256, 256^2 x 512) but 15 % slower
-        // on the upsampling convs, whose residual epilogue reads the shortcut.
         if (p.N <= 64) return launch_conv<128, 64, 2, 2, 2, 3>(p, s);
-        if (p.conv == 2) return launch_conv<128, 128, 2, 2, 2, 1>(p, s);
-        return launch_conv<128, 128, 2, 2, 2, 3>(p, s);
+        // A round of 256 workgroups of 256x256 takes 1.85 of a round of 512 of
+        // 128x128 (us, before -> after: 512^2 x 256 conv1 364 -> 337, conv2 391 ->
+        // 370; 256^2 x 512 340 -> 301, 348 -> 323; onto 512^2 x 256 820 -> 700).
+        if (rounds(256, 256, 256) * 185 < rounds(128, 128, 512) * 100)
+            return launch_conv<256, 256, 2, 4, 2, 2>(p, s);
+        // (1024^2 x 128: conv1 433 -> 426, conv2 467 -> 460; the upsampling conv, whose
+        // residual epilogue reads the shortcut, 944 -> 897 with 8 waves)
+        if (p.conv == 2) return launch_conv<128, 128, 4, 2, 2, 2>(p, s);
+        return launch_conv<128, 128, 2, 2, 2, 2>(p, s);
     }
     // Tile choice from sweeps on MI355X with cold weights (each GEMM's weights
     // come from HBM, as in the 28-block forward).  Every CU pulls at most
@@ -1061,10 +1087,18 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     //  * at most 5 row (or column) tiles of 128 against >= 128 of the other
     //    (the step's cross K 600 x 32256 and V^T 32256 x 600): 128x128 tiles
     //    of 8 waves (4 x 2, 32 x 64 per wave): 67.4 -> 60.0 us and 63.2 -> 60.8 us;
+    //  * stores and the q|k|v split with more 128x128 tiles than slots: 256x256
+    //    tiles where their rounds of 256 workgroups, 1.82 of a round of 512 of
+    //    128x128 each (128x192: 1.41), come to less (us, before -> after: 738 x
+    //    18432 x 2304 gate | up 90 -> 75; 4096 x 3456 x 1152 48.4 -> 42.5; 8192 x
+    //    5760 x 1152 135 -> 129; 8192^3 945 -> 1105 TFLOP/s).  Their waves read
+    //    half of the LDS bytes per product of 64 x 64 ones;
     //  * otherwise 128x128 tiles with two stages, two workgroups per CU.
-    //  The QKV-split GEMM (both sizes) and, with 128x192 tiles, the residual
-    //  GEMMs with K <= 1152 use workgroups of 8 waves (4 x 2): the forward at
-    //  16384 rows per branch 54.00 -> 53.66 ms, at 1024 rows 5.089 -> 5.081 ms.
+    //  The last four use schedule 2 (against 1, 16384 rows: 128x192 stores and
+    //  q|k|v 260 -> 256 and 163 -> 156 us, K = 2880 residuals 138 -> 136.5; 128x128
+    //  q|k|v of two 2048-row launches 45.2 -> 43.0), except that the 128x192
+    //  residual GEMMs with K <= 1152 keep 8 waves (4 x 2) and schedule 1 (72 us
+    //  against 74).
     // (tile counts are scaled by the launches that share the CUs, p.co, and
     // by the products of a batched launch)
     // Grids of few tiles leave most CUs idle and each workgroup with a chain of
@@ -1109,14 +1143,17 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     const int64_t t192 = p.N % 192 == 0 ? tm128 * (p.N / 192) * co : 0;
     constexpr int64_t kSlots = 512;
     const bool one_round192 = p.mode == kGemmStore && p.N >= 3456 && t192 > 0 && t192 <= kSlots && t128 > kSlots;
+    if (t128 > kSlots && (p.mode == kGemmStore || p.mode == kGemmQKV)) {
+        const int64_t c256 = rounds(256, 256, 256) * 182, c128 = rounds(128, 128, kSlots) * 100;
+        if (c256 < c128 && (p.N % 192 || c256 < rounds(128, 192, kSlots) * 141)) return launch256(p, s);
+    }
     if (!one_round192 && co == 1 && std::min(tm128, tn128) <= 5 && std::max(tm128, tn128) >= 128)
         return launch<128, 128, 4, 2, 2, 1>(p, s);
     if (t192 >= kSlots * 3 / 2 || one_round192) {
-        if (p.mode == kGemmQKV || (p.mode == kGemmResidual && p.K <= 1152)) return launch<128, 192, 4, 2, 2, 1>(p, s);
-        return launch<128, 192, 2, 2, 2, 1>(p, s);
+        if (p.mode == kGemmResidual && p.K <= 1152) return launch<128, 192, 4, 2, 2, 1>(p, s);
+        return launch<128, 192, 2, 2, 2, 2>(p, s);
     }
-    if (p.mode == kGemmQKV) return launch<128, 128, 4, 2, 2, 1>(p, s);
-    return launch<128, 128, 2, 2, 2, 1>(p, s);
+    return launch<128, 128, 2, 2, 2, 2>(p, s);
 }
 
 }  // namespace sana

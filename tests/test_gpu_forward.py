@@ -131,6 +131,20 @@ def test_step_device_matches_context_then_forward(full_model, masked):
         assert np.array_equal(got, ref)
 
 
+def test_block_256_tiles(full_model):
+    """One block on 16 x 256 tokens at once (256x256 tiles for the q|k|v split)
+    against pairs of them (k-groups of small tiles): the fp32 sums differ in
+    order, so a few of the 11-bit fp16 operands round the other way."""
+    m, d = full_model
+    x, ctx, tmod = O.randn((16, 256, 1152), 21), O.randn((16, 300, 1152), 22), 0.1 * O.randn((16, 6 * 1152), 23)
+    d.set_context(ctx, projected=True)
+    got = d.run_blocks(0, 1, x, tmod)
+    for i in range(0, 16, 2):
+        d.set_context(ctx[i:i + 2], projected=True)
+        ref = d.run_blocks(0, 1, x[i:i + 2], tmod[i:i + 2])
+        assert rel_l2(got[i:i + 2] - x[i:i + 2], ref - x[i:i + 2]) < 2.0 ** -11
+
+
 def test_forward_deterministic(full_model):
     m, d = full_model
     latent = O.randn((1, 32, 32, 32), 42)

@@ -97,6 +97,45 @@ def test_gemm_k_groups(L, M, N, K):
     assert (np.abs(host(o16) - rx) <= tol + 2.0 ** -11 * np.abs(rx) + 2.0 ** -24).all()
 
 
+# more 128x128 tiles than two rounds hold and few enough 256x256 ones: the 8-wave
+# 256x256 kernel (one k-tile, few, many; ragged rows and columns; padded strides)
+@pytest.mark.parametrize("act,M,N,K,pad", [(0, 3970, 4096, 64, 0), (1, 3841, 4088, 448, 8), (2, 3841, 4090, 128, 8),
+                                           (0, 4096, 4090, 192, 0)])
+def test_gemm_256_tiles(L, act, M, N, K, pad):
+    """fp16 and fp32 stores equal 512-row slices (smaller tiles, the same k order)
+    bit for bit; sampled rows against fp64 (activation applied to fp32 sums)."""
+    rng = np.random.default_rng(M + N + K)
+    lda, ldw, ldo = K + pad, K + pad, N + pad
+    A, W = f16(rng.standard_normal((M, lda))), f16(rng.standard_normal((N, ldw)) * 0.05)
+    bias = rng.standard_normal(N).astype(np.float32)
+    dA, dW, db = dev(A, torch.float16), dev(W, torch.float16), dev(bias, torch.float32)
+
+    def run(r0, r1, f32):
+        o16 = torch.full((r1 - r0, ldo), float("nan"), device="cuda", dtype=torch.float16)
+        o32 = torch.full((r1 - r0, ldo), float("nan"), device="cuda", dtype=torch.float32) if f32 else None
+        L.check(L.lib().sana_hip_gemm(dA[r0:].data_ptr(), lda, dW.data_ptr(), ldw, r1 - r0, N, K, db.data_ptr(), act,
+                                      o16.data_ptr(), ldo, o32.data_ptr() if f32 else None, ldo, stream()))
+        assert torch.isnan(o16[:, N:]).all()
+        return o16[:, :N], o32[:, :N] if f32 else None
+
+    w16, _ = run(0, M, False)
+    x16, x32 = run(0, M, True)
+    for r0 in range(0, M, 512):
+        p16, p32 = run(r0, min(M, r0 + 512), True)
+        assert torch.equal(w16[r0:r0 + 512], p16) and torch.equal(x16[r0:r0 + 512], p16)
+        assert torch.equal(x32[r0:r0 + 512], p32)
+    rows = np.r_[0, 127, 255, 256, M - 1]
+    ref = A[rows, :K].astype(np.float64) @ W[:, :K].astype(np.float64).T + bias
+    mag = np.abs(A[rows, :K]).astype(np.float64) @ np.abs(W[:, :K]).astype(np.float64).T + np.abs(bias)
+    if act == 1:
+        ref = ref / (1 + np.exp(-ref))
+    elif act == 2:
+        ref = 0.5 * ref * (1 + np.tanh(np.sqrt(2 / np.pi) * (ref + 0.044715 * ref ** 3)))
+    # sums as in test_gemm_k_groups; the activations' slope is below 1.13, their own error a few ulp
+    bound = 1.13 * (K + 8) * 2.0 ** -24 * mag + 16 * 2.0 ** -24 * np.abs(mag)
+    assert (np.abs(host(x32)[rows] - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("M,N,K", GEMM_SHAPES)
 def test_gemm_store(L, M, N, K):
     rng = np.random.default_rng(M * 7 + N)

@@ -82,6 +82,26 @@ def test_batch_matches_single():
         dev.close()
 
 
+def test_256_tile_convs_equal_smaller_tiles():
+    """The 3x3 convs of 182 x 202 pixels and 256 channels (plain, upsampling,
+    conv_in) run on 256x256 tiles, those of the latent's upper part on 128x128
+    ones, with the same k order: pixels beyond the convs' reach from
+    the cut (1 + 6 latent rows, 1 + 6 + 1 image rows) are bit-identical."""
+    ora, dev = build(dict(channels=(256, 256), attn=(False, False)))
+    try:
+        lat = O.randn((1, 32, 91, 101), 11)
+        whole, cut = dev.decode(lat), dev.decode(lat[:, :, :52])
+        assert np.isfinite(whole).all()
+        assert np.array_equal(whole[:, :, :80], cut[:, :, :80])
+        dev2 = build(dict(channels=(256,), attn=(False,)))[1]
+        lat = O.randn((1, 32, 182, 202), 12)
+        whole, cut = dev2.decode(lat), dev2.decode(lat[:, :, :110])
+        assert np.array_equal(whole[:, :, :100], cut[:, :, :100])
+        dev2.close()
+    finally:
+        dev.close()
+
+
 def test_rejects_bad_input():
     import sana_dit
     with pytest.raises(sana_dit.SanaError):
