@@ -28,6 +28,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/sana_dit.h"
@@ -104,60 +105,87 @@ __global__ void vae_zero_border_kernel(f16 * __restrict__ buf, int B, int H, int
 // Per-pixel RMSNorm over channels (rms_norm_4d_channelwise,
 // src/vae_ops.cpp:476-560): v = x / sqrt(mean(x^2) + eps) * w + b, then the
 // block's residual (+ res, src/vae_ops.cpp:581,605,804) and the decoder's
-// final ReLU (src/vae.cpp:320).  One wave per pixel; fp32 out and/or fp16 out
-// (plain, or into the interior of a bordered H x W grid when pad != 0).
-template <int NC4>  // float4 chunks per lane, C <= 256 * NC4
+// final ReLU (src/vae.cpp:320).  fp32 out and/or fp16 out (plain, or into the
+// interior of a bordered H x W grid when pad != 0); out32 may be res.
+// Bound by memory: LPR lanes take a row (32 up to 128 channels, so none idles)
+// and a wave takes U times 64 / LPR rows, all of whose loads (x, residual) are
+// requested before the first sum (one wave and one row at a time before): us,
+// 1024^2 x 128 with residual 402 -> 330, 512^2 x 256 221 -> 161, 256^2 x 512 39 -> 37.
+template <int NC4, int LPR, int U>  // float4 chunks per lane, C <= 4 * LPR * NC4
 __global__ __launch_bounds__(256) void vae_rmsnorm_kernel(const float * __restrict__ x, int C, int P,
                                                           const float * __restrict__ w,
                                                           const float * __restrict__ bias,
-                                                          const float * __restrict__ res, int relu, float eps,
-                                                          float * __restrict__ out32, f16 * __restrict__ out16,
-                                                          int pad, int H, int W) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (row >= P) return;
+                                                          const float * res, int relu, float eps, float * out32,
+                                                          f16 * __restrict__ out16, int pad, int H, int W) {
+    constexpr int RPW = 64 / LPR;
+    const int lane = threadIdx.x & 63, sub = lane % LPR;
+    const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (RPW * U) + lane / LPR;
     const int n4 = C >> 2;
-    const float4 * xr = reinterpret_cast<const float4 *>(x + (int64_t)row * C);
-    float4 v[NC4];
-    float ss = 0.0f;
+    float4 v[U][NC4], r[U][NC4], g[NC4], bb[NC4];
+    // rows past P read the last one and columns past C the last chunk; neither is stored
 #pragma unroll
-    for (int i = 0; i < NC4; ++i) {
-        const int c4 = lane + 64 * i;
-        if (c4 < n4) {
-            v[i] = xr[c4];
-            ss += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
-        } else {
-            v[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-    }
-    const float inv = 1.0f / sqrtf(wave_sum(ss) * (1.0f / (float)C) + eps);
-    int64_t orow = row;
-    if (pad) {
-        const int hw = H * W, img = row / hw, rem = row - img * hw, yy = rem / W, xx = rem - yy * W;
-        orow = ((int64_t)img * (H + 2) + yy + 1) * (W + 2) + xx + 1;
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < NC4; ++i)
+            v[u][i] = reinterpret_cast<const float4 *>(x + (int64_t)min(row0 + u * RPW, P - 1) * C)[min(sub + LPR * i, n4 - 1)];
+    if (res) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < NC4; ++i)
+                r[u][i] = reinterpret_cast<const float4 *>(res + (int64_t)min(row0 + u * RPW, P - 1) * C)[min(sub + LPR * i, n4 - 1)];
     }
 #pragma unroll
     for (int i = 0; i < NC4; ++i) {
-        const int c4 = lane + 64 * i;
-        if (c4 >= n4) continue;
-        const float4 g = reinterpret_cast<const float4 *>(w)[c4];
-        const float4 bb = bias ? reinterpret_cast<const float4 *>(bias)[c4] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        float o[4] = {v[i].x * inv * g.x + bb.x, v[i].y * inv * g.y + bb.y, v[i].z * inv * g.z + bb.z,
-                      v[i].w * inv * g.w + bb.w};
-        if (res) {
-            const float4 r = reinterpret_cast<const float4 *>(res + (int64_t)row * C)[c4];
-            o[0] += r.x; o[1] += r.y; o[2] += r.z; o[3] += r.w;
-        }
-        if (relu) {
+        const int c4 = min(sub + LPR * i, n4 - 1);
+        g[i] = reinterpret_cast<const float4 *>(w)[c4];
+        bb[i] = bias ? reinterpret_cast<const float4 *>(bias)[c4] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    float ss[U];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = fmaxf(o[e], 0.0f);
-        }
-        if (out32) reinterpret_cast<float4 *>(out32 + (int64_t)row * C)[c4] = make_float4(o[0], o[1], o[2], o[3]);
-        if (out16) {
-            f16x4 h;
+    for (int u = 0; u < U; ++u) {
+        ss[u] = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = (f16)o[e];
-            *reinterpret_cast<f16x4 *>(out16 + orow * C + 4 * c4) = h;
+        for (int i = 0; i < NC4; ++i) {
+            const float4 & q = v[u][i];
+            const float t = (q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w);
+            ss[u] += sub + LPR * i < n4 ? t : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int m = LPR / 2; m; m >>= 1)
+#pragma unroll
+        for (int u = 0; u < U; ++u) ss[u] += __shfl_xor(ss[u], m, 64);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int row = row0 + u * RPW;
+        if (row >= P) break;
+        const float inv = 1.0f / sqrtf(ss[u] * (1.0f / (float)C) + eps);
+        int64_t orow = row;
+        if (pad) {
+            const int hw = H * W, img = row / hw, rem = row - img * hw, yy = rem / W, xx = rem - yy * W;
+            orow = ((int64_t)img * (H + 2) + yy + 1) * (W + 2) + xx + 1;
+        }
+#pragma unroll
+        for (int i = 0; i < NC4; ++i) {
+            const int c4 = sub + LPR * i;
+            if (c4 >= n4) continue;
+            float o[4] = {v[u][i].x * inv * g[i].x + bb[i].x, v[u][i].y * inv * g[i].y + bb[i].y,
+                          v[u][i].z * inv * g[i].z + bb[i].z, v[u][i].w * inv * g[i].w + bb[i].w};
+            if (res) {
+                o[0] += r[u][i].x; o[1] += r[u][i].y; o[2] += r[u][i].z; o[3] += r[u][i].w;
+            }
+            if (relu) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = fmaxf(o[e], 0.0f);
+            }
+            if (out32) reinterpret_cast<float4 *>(out32 + (int64_t)row * C)[c4] = make_float4(o[0], o[1], o[2], o[3]);
+            if (out16) {
+                f16x4 h;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h[e] = (f16)o[e];
+                *reinterpret_cast<f16x4 *>(out16 + orow * C + 4 * c4) = h;
+            }
         }
     }
 }
@@ -165,36 +193,75 @@ __global__ __launch_bounds__(256) void vae_rmsnorm_kernel(const float * __restri
 // Depthwise 5x5, zero padding, no bias (the multiscale proj_in,
 // depthwise_conv5x5_process_plane src/common_ops.cpp:628-649): taps in (ky, kx)
 // order.  Token-major fp16 in/out [P][C], tap-major fp32 weights [25][C]; one
-// thread per (pixel, 8 channels).
+// thread per (XS pixels of a row, 8 channels).  XS = 4: the columns of a kernel
+// row are loaded once for four outputs, as are its weights (per pixel it is 25
+// input and 50 weight chunks of 16 bytes an output, and the caches' rate bounds
+// it).  XS = 1 for grids too small to hide latency otherwise: all taps are
+// requested at once.  Taps outside the image are loaded from its edge and not
+// added.  The nine of a 1024 px decode (128^2 x 1536 to 32^2 x 3072) 676 -> 349 us
+// (without the second variant 451).
+template <int XS>
 __global__ __launch_bounds__(256) void vae_dw5x5_kernel(const f16 * __restrict__ in, const float * __restrict__ w,
                                                         f16 * __restrict__ out, int B, int H, int W, int C) {
-    const int G = C / 8;
+    const int G = C / 8, strips = (W + XS - 1) / XS;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)B * H * W * G) return;
+    if (i >= (int64_t)B * H * strips * G) return;
     const int g = (int)(i % G);
-    const int64_t p = i / G;
-    const int xx = (int)(p % W), yy = (int)((p / W) % H), b = (int)(p / ((int64_t)W * H));
-    float acc[8];
+    const int64_t row = i / G / strips;  // image row b * H + y
+    const int x0 = (int)(i / G - row * strips) * XS, yy = (int)(row % H);
+    const f16 * src = in + (row * W + x0) * C + g * 8;
+    f16 * dst = out + (row * W + x0) * C + g * 8;
+    float acc[XS][8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-    for (int ky = 0; ky < 5; ++ky) {
-        const int iy = yy + ky - 2;
-        if (iy < 0 || iy >= H) continue;
-        for (int kx = 0; kx < 5; ++kx) {
-            const int ix = xx + kx - 2;
-            if (ix < 0 || ix >= W) continue;
-            const f16x8 v = *reinterpret_cast<const f16x8 *>(in + (((int64_t)b * H + iy) * W + ix) * C + g * 8);
-            const float4 * wp = reinterpret_cast<const float4 *>(w + (ky * 5 + kx) * C + g * 8);
-            const float4 w0 = wp[0], w1 = wp[1];
-            const float wk[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+    for (int k = 0; k < XS; ++k)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] += (float)v[e] * wk[e];
+        for (int e = 0; e < 8; ++e) acc[k][e] = 0.0f;
+    auto taps = [&](auto edge) {
+#pragma unroll (XS == 1 ? 5 : 1)
+        for (int ky = 0; ky < 5; ++ky) {
+            const int dy = ky - 2;
+            const bool row_in = !edge || (yy + dy >= 0 && yy + dy < H);
+            f16x8 v[XS + 4];
+            float4 wk[5][2];
+#pragma unroll
+            for (int c = 0; c < XS + 4; ++c) {
+                const int ry = edge ? min(max(yy + dy, 0), H - 1) - yy : dy;
+                const int rx = edge ? min(max(x0 + c - 2, 0), W - 1) - x0 : c - 2;
+                v[c] = *reinterpret_cast<const f16x8 *>(src + ((int64_t)ry * W + rx) * C);
+            }
+#pragma unroll
+            for (int kx = 0; kx < 5; ++kx) {
+                const float4 * wp = reinterpret_cast<const float4 *>(w + (ky * 5 + kx) * C + g * 8);
+                wk[kx][0] = wp[0];
+                wk[kx][1] = wp[1];
+            }
+#pragma unroll
+            for (int kx = 0; kx < 5; ++kx) {
+                const float t[8] = {wk[kx][0].x, wk[kx][0].y, wk[kx][0].z, wk[kx][0].w,
+                                    wk[kx][1].x, wk[kx][1].y, wk[kx][1].z, wk[kx][1].w};
+#pragma unroll
+                for (int k = 0; k < XS; ++k) {
+                    const int ix = x0 + k + kx - 2;
+                    const bool in_image = !edge || (row_in && ix >= 0 && ix < W);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float sum = acc[k][e] + (float)v[k + kx][e] * t[e];
+                        acc[k][e] = in_image ? sum : acc[k][e];
+                    }
+                }
+            }
         }
-    }
-    f16x8 o;
+    };
+    if (x0 >= 2 && x0 + XS + 2 <= W && yy >= 2 && yy + 2 < H) taps(std::false_type{});
+    else taps(std::true_type{});
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = (f16)acc[e];
-    *reinterpret_cast<f16x8 *>(out + p * C + g * 8) = o;
+    for (int k = 0; k < XS; ++k) {
+        if (x0 + k >= W) break;
+        f16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (f16)acc[k][e];
+        *reinterpret_cast<f16x8 *>(dst + k * C) = o;
+    }
 }
 
 // Grouped 1x1 conv with groups of 32 channels (the multiscale proj_out,
@@ -536,15 +603,16 @@ void gemm_conv(int conv, const half_t * A, int64_t cin, const DevMem & W, int64_
 
 void rmsnorm(const float * x, int64_t C, int64_t P, const DevMem & w, const DevMem * b, const float * res, bool relu,
              float * out32, half_t * out16, bool pad, int64_t H, int64_t W, hipStream_t s) {
-    const dim3 g((unsigned)((P + 3) / 4)), t(256);
     f16 * o16 = reinterpret_cast<f16 *>(out16);
     const float * bp = b ? b->as<float>() : nullptr;
-#define SANA_VAE_RMS(n4) \
-    hipLaunchKernelGGL((vae_rmsnorm_kernel<n4>), g, t, 0, s, x, (int)C, (int)P, w.as<float>(), bp, res, relu ? 1 : 0, \
-                       1e-5f, out32, o16, pad ? 1 : 0, (int)H, (int)W)
-    if (C <= 256) SANA_VAE_RMS(1);
-    else if (C <= 512) SANA_VAE_RMS(2);
-    else SANA_VAE_RMS(4);
+#define SANA_VAE_RMS(n4, lpr, u)                                                                                  \
+    hipLaunchKernelGGL((vae_rmsnorm_kernel<n4, lpr, u>), dim3(blocks_for(P, 4 * (64 / lpr) * u)), dim3(256), 0, s, \
+                       x, (int)C, (int)P, w.as<float>(), bp, res, relu ? 1 : 0, 1e-5f, out32, o16, pad ? 1 : 0,   \
+                       (int)H, (int)W)
+    if (C <= 128) SANA_VAE_RMS(1, 32, 4);
+    else if (C <= 256) SANA_VAE_RMS(1, 64, 4);
+    else if (C <= 512) SANA_VAE_RMS(2, 64, 2);
+    else SANA_VAE_RMS(4, 64, 1);
 #undef SANA_VAE_RMS
     launch_check(hipGetLastError(), "vae rmsnorm");
 }
@@ -666,8 +734,11 @@ void decode(sana_vae * v, const float * lat, int64_t B, int64_t h, int64_t w, fl
                 gemm_plain(v->a16.as<half_t>(), C, a.wqkv, P, 3 * C, C, nullptr, sana::kActNone, qkv, 3 * C, nullptr,
                            0, s, B);
                 {
-                    const int64_t n = P * (3 * C / 8);
-                    hipLaunchKernelGGL(vae_dw5x5_kernel, dim3(blocks_for(n)), dim3(256), 0, s,
+                    const int64_t n4 = B * H * ((W + 3) / 4) * (3 * C / 8);
+                    // (2 waves per SIMD)
+                    const bool strips = n4 >= 2 * 64 * 1024;
+                    const auto k = strips ? vae_dw5x5_kernel<4> : vae_dw5x5_kernel<1>;
+                    hipLaunchKernelGGL(k, dim3(blocks_for(strips ? n4 : P * (3 * C / 8))), dim3(256), 0, s,
                                        reinterpret_cast<const f16 *>(qkv), a.dw5.as<float>(), v->dw16.as<f16>(), (int)B,
                                        (int)H, (int)W, (int)(3 * C));
                     launch_check(hipGetLastError(), "vae dw5x5");

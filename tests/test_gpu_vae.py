@@ -59,6 +59,18 @@ def test_decode_vs_oracle(name, shape):
         dev.close()
 
 
+# widths around the depthwise 5x5's strips (4 pixels and 2 of border each side)
+# and row counts that leave the norms' last group of rows partial
+@pytest.mark.parametrize("shape", [(1, 32, 1, 1), (1, 32, 3, 5), (2, 32, 5, 8), (1, 32, 6, 11), (1, 32, 2, 18)])
+def test_attention_level_widths_vs_oracle(shape):
+    ora, dev = build(CONFIGS["evit1"])
+    try:
+        lat = O.randn(shape, 13)
+        assert rel_l2(dev.decode(lat), ora.decode(lat)) < TOL
+    finally:
+        dev.close()
+
+
 def test_small_decode_vs_reference_fixture():
     fx = np.load(os.path.join(GOLDEN, "vae_small.npz"), allow_pickle=False)
     ora, dev = build(CONFIGS["small"])
