@@ -60,8 +60,8 @@ constexpr int kTK = 32;
 //
 // Measured on MI355X: 2048 x 1152 x 1152 65 us (84 TFLOP/s); with the other
 // kernels of this file the fp32 self-attention block (2 x 1024 tokens, four
-// such products) went from 1316 to 314 us and the cross-attention block (2 x
-// 256 tokens, 300 keys) from 787 to 140 us, against a 64 x 64 tile with
+// such products) went from 1316 to 288 us and the cross-attention block (2 x
+// 256 tokens, 300 keys) from 787 to 139 us, against a 64 x 64 tile with
 // single-buffered 16-deep k-tiles and two barriers each.
 template <int BM, int BN, bool BT, int VA, int VB>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(OpGemm p, int tiles_n) {

@@ -109,8 +109,9 @@ __global__ void vae_zero_border_kernel(f16 * __restrict__ buf, int B, int H, int
 // interior of a bordered H x W grid when pad != 0); out32 may be res.
 // Bound by memory: LPR lanes take a row (32 up to 128 channels, so none idles)
 // and a wave takes U times 64 / LPR rows, all of whose loads (x, residual) are
-// requested before the first sum (one wave and one row at a time before): us,
-// 1024^2 x 128 with residual 402 -> 330, 512^2 x 256 221 -> 161, 256^2 x 512 39 -> 37.
+// requested before the first sum (one wave and one row at a time before).  A
+// 1024 px decode's four launches at 1024^2 x 128 and three at 512^2 x 256: 2104
+// -> 1625 us (5.4 TB/s); nine at 256^2 x 512 351 -> 331.
 template <int NC4, int LPR, int U>  // float4 chunks per lane, C <= 4 * LPR * NC4
 __global__ __launch_bounds__(256) void vae_rmsnorm_kernel(const float * __restrict__ x, int C, int P,
                                                           const float * __restrict__ w,
