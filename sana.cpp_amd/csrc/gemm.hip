@@ -114,10 +114,10 @@ SANA_DEV void wait_stages(int keep) {
 // CONV: 0 plain A rows; 1 implicit 3x3 conv over a zero-bordered NHWC input;
 // 2 the same over the nearest-2x upsample of the input (GemmParams::conv).
 template <int BM, int BN, int WM, int WN, int STAGES, int MODE, int SCHED, int ACT, int CONV = 0, int KG = 1,
-          int SEG = 1>
+          bool FOLD = false>
 __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in) {
     using G = Cfg<BM, BN, WM, WN, STAGES, KG>;
-    static_assert((KG == 1 || SCHED == 1) && (SEG == 1 || (KG == 1 && SCHED != 2)), "schedule");
+    static_assert((KG == 1 || SCHED == 1) && (!FOLD || (KG == 1 && SCHED != 2)), "schedule");
     // product blockIdx.y of a batched launch (plain stores only)
     GemmParams p = p_in;
     if constexpr (MODE == kGemmStore && CONV == 0) {
@@ -266,20 +266,22 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in
             for (int j = 0; j < G::TN; ++j) acc[i][j] = mfma_32x32x16(bf[buf][j], af[buf][i], acc[i][j]);
     };
 
-    // SEG > 1: the sums of SEG runs of consecutive k-tiles, added in run order --
-    // the order of SEG k-groups, so that kernels of either kind agree bit for bit.
-    f32x16 tot[SEG > 1 ? G::TM : 1][SEG > 1 ? G::TN : 1];
-    if constexpr (SEG > 1) {
+    // FOLD: the sums of p.k_runs runs of consecutive k-tiles, added in run order --
+    // the order of that many k-groups, so that kernels of either kind agree bit
+    // for bit.
+    f32x16 tot[FOLD ? G::TM : 1][FOLD ? G::TN : 1];
+    if constexpr (FOLD) {
 #pragma unroll
         for (int i = 0; i < G::TM; ++i)
 #pragma unroll
             for (int j = 0; j < G::TN; ++j) tot[i][j] = acc[i][j];
     }
-    int run_left = (KT + SEG - 1) / SEG;  // k-tiles of the current run still to come
+    const int run = FOLD ? (KT + p.k_runs - 1) / p.k_runs : KT;
+    int run_left = run;  // k-tiles of the current run still to come
     auto fold = [&]() {
-        if constexpr (SEG > 1) {
+        if constexpr (FOLD) {
             if (--run_left) return;
-            run_left = (KT + SEG - 1) / SEG;
+            run_left = run;
 #pragma unroll
             for (int i = 0; i < G::TM; ++i)
 #pragma unroll
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_kernel(GemmParams p_in
         }
     }
 
-    if constexpr (SEG > 1) {  // the last run (all zeros where it was folded above)
+    if constexpr (FOLD) {  // the last run (all zeros where it was folded above)
 #pragma unroll
         for (int i = 0; i < G::TM; ++i)
 #pragma unroll
@@ -904,19 +906,19 @@ bool set_lds_limit(const void * k, size_t lds) {
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int MODE, int SCHED, int ACT, int CONV = 0, int KG = 1,
-          int SEG = 1>
+          bool FOLD = false>
 hipError_t launch_mode(const GemmParams & p, int tiles, hipStream_t s) {
     using G = Cfg<BM, BN, WM, WN, STAGES, KG>;
     static const bool attr = set_lds_limit(
-        reinterpret_cast<const void *>(&gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV, KG, SEG>), G::LDS_BYTES);
+        reinterpret_cast<const void *>(&gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV, KG, FOLD>), G::LDS_BYTES);
     (void)attr;
     static const std::string name = "gemm_kernel<" + std::to_string(BM) + ", " + std::to_string(BN) + ", " +
                                     std::to_string(WM) + ", " + std::to_string(WN) + ", " + std::to_string(STAGES) +
                                     ", " + std::to_string(MODE) + ", " + std::to_string(SCHED) + ", " +
                                     std::to_string(ACT) + ", " + std::to_string(CONV) + ", " +
-                                    std::to_string(KG) + ", " + std::to_string(SEG) + ">";
+                                    std::to_string(KG) + (FOLD ? ", true>" : ", false>");
     note_kernel(name.c_str());
-    hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV, KG, SEG>), dim3(tiles, p.batch), dim3(G::NT),
+    hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, STAGES, MODE, SCHED, ACT, CONV, KG, FOLD>), dim3(tiles, p.batch), dim3(G::NT),
                        G::LDS_BYTES, s, p);
     return hipGetLastError();
 }
@@ -937,33 +939,36 @@ hipError_t launch_conv(const GemmParams & p, hipStream_t s) {
     return launch_conv_mode<BM, BN, WM, WN, STAGES, SCHED, 1>(p, s);
 }
 
-// Few-tile grids: k-groups (stores, residual updates, the q|k|v split).
-template <int BM, int BN, int WM, int WN, int STAGES, int KG>
-hipError_t launch_kg(const GemmParams & p, hipStream_t s) {
-    const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-    if (p.mode == kGemmResidual)
-        return launch_mode<BM, BN, WM, WN, STAGES, kGemmResidual, 1, kActNone, 0, KG>(p, tiles, s);
-    if (p.mode == kGemmQKV) return launch_mode<BM, BN, WM, WN, STAGES, kGemmQKV, 1, kActNone, 0, KG>(p, tiles, s);
-    if (p.act == kActSilu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActSilu, 0, KG>(p, tiles, s);
-    if (p.act == kActGelu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActGelu, 0, KG>(p, tiles, s);
-    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActNone, 0, KG>(p, tiles, s);
-}
-
-// Plain stores whose k sums are four runs added in order (GemmParams::k_runs):
-// four k-groups, or one group that folds its sums.
+// Sums of several runs of k (GemmParams::k_runs): KG groups of waves, one run
+// each, or (KG = 1) one group that folds its sums.  Stores, residual updates and
+// the q|k|v split.
 template <int BM, int BN, int WM, int WN, int STAGES, int SCHED, int KG>
 hipError_t launch_runs(const GemmParams & p, hipStream_t s) {
-    const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, SCHED, kActNone, 0, KG, 4 / KG>(p, tiles, s);
-}
-
-template <int BM, int BN, int WM, int WN, int STAGES, int CONV, int KG>
-hipError_t launch_conv_kg(const GemmParams & p, hipStream_t s) {
+    constexpr bool F = KG == 1;
     const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
     if (p.mode == kGemmResidual)
-        return launch_mode<BM, BN, WM, WN, STAGES, kGemmResidual, 1, kActNone, CONV, KG>(p, tiles, s);
-    if (p.act == kActSilu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActSilu, CONV, KG>(p, tiles, s);
-    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, 1, kActNone, CONV, KG>(p, tiles, s);
+        return launch_mode<BM, BN, WM, WN, STAGES, kGemmResidual, SCHED, kActNone, 0, KG, F>(p, tiles, s);
+    if (p.mode == kGemmQKV) return launch_mode<BM, BN, WM, WN, STAGES, kGemmQKV, SCHED, kActNone, 0, KG, F>(p, tiles, s);
+    if (p.act == kActSilu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, SCHED, kActSilu, 0, KG, F>(p, tiles, s);
+    if (p.act == kActGelu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, SCHED, kActGelu, 0, KG, F>(p, tiles, s);
+    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, SCHED, kActNone, 0, KG, F>(p, tiles, s);
+}
+
+// The same for the 3x3 convolutions.
+template <int BM, int BN, int WM, int WN, int STAGES, int SCHED, int CONV, int KG>
+hipError_t launch_conv_runs_mode(const GemmParams & p, hipStream_t s) {
+    constexpr bool F = KG == 1;
+    const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+    if (p.mode == kGemmResidual)
+        return launch_mode<BM, BN, WM, WN, STAGES, kGemmResidual, SCHED, kActNone, CONV, KG, F>(p, tiles, s);
+    if (p.act == kActSilu) return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, SCHED, kActSilu, CONV, KG, F>(p, tiles, s);
+    return launch_mode<BM, BN, WM, WN, STAGES, kGemmStore, SCHED, kActNone, CONV, KG, F>(p, tiles, s);
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES, int SCHED, int KG>
+hipError_t launch_conv_runs(const GemmParams & p, hipStream_t s) {
+    if (p.conv == 2) return launch_conv_runs_mode<BM, BN, WM, WN, STAGES, SCHED, 2, KG>(p, s);
+    return launch_conv_runs_mode<BM, BN, WM, WN, STAGES, SCHED, 1, KG>(p, s);
 }
 
 // 256 x 256 tiles (8 waves of 128 x 64, one workgroup per CU): stores and the q|k|v split.
@@ -1040,9 +1045,16 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     if (p.bias) vec = vec && (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0;
     p.vec = vec ? 1 : 0;
     const int64_t co = std::max(p.co, 1) * (int64_t)p.batch;
-    // tiles of the rows that decide the order of the k sums
-    const int64_t rows = p.order_rows > 0 ? p.order_rows : p.M;
-    auto grid = [&](int bm, int bn) { return (rows + bm - 1) / bm * ((p.N + bn - 1) / bn) * co; };
+    auto grid = [&](int bm, int bn) { return ((int64_t)p.M + bm - 1) / bm * ((p.N + bn - 1) / bn) * co; };
+    // The order of the k sums follows from the rows that decide it alone
+    // (GemmParams::order_rows), the tiles below from the launch's own rows.
+    if (p.k_runs == 1 && p.order_rows >= 0 &&
+        (p.conv || (p.K >= 512 && p.batch == 1 && p.mode != kGemmVT && p.act != kActGeglu))) {
+        const int64_t rows = p.order_rows > 0 ? p.order_rows : p.M;
+        auto order = [&](int bm, int bn) { return (rows + bm - 1) / bm * ((p.N + bn - 1) / bn) * co; };
+        if (order(32, 64) <= 288 || (!p.conv && order(32, 32) <= 256)) p.k_runs = 4;
+        else if (order(64, 64) <= (p.conv ? 320 : 256)) p.k_runs = 2;
+    }
     // Rounds (in 1/64) of `slots` workgroups at a time that bm x bn tiles of all
     // rows take; launches that share the CUs fill each other's last round.
     auto rounds = [&](int bm, int bn, int64_t slots) {
@@ -1050,10 +1062,14 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
         return co > 1 ? std::max<int64_t>(64, t * 64 / slots) : (t + slots - 1) / slots * 64;
     };
     if (p.conv) {
-        if (grid(32, 64) <= 288)
-            return p.conv == 2 ? launch_conv_kg<32, 64, 1, 2, 3, 2, 4>(p, s) : launch_conv_kg<32, 64, 1, 2, 3, 1, 4>(p, s);
-        if (grid(64, 64) <= 320)
-            return p.conv == 2 ? launch_conv_kg<64, 64, 2, 2, 4, 2, 2>(p, s) : launch_conv_kg<64, 64, 2, 2, 4, 1, 2>(p, s);
+        if (p.k_runs == 4 && grid(32, 64) <= 288) return launch_conv_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
+        if (p.k_runs == 4 && grid(64, 64) <= 256) return launch_conv_runs<64, 64, 2, 2, 2, 1, 4>(p, s);
+        if (p.k_runs == 2 && grid(64, 64) <= 320) return launch_conv_runs<64, 64, 2, 2, 4, 1, 2>(p, s);
+        if (p.k_runs > 1) {
+            if (p.N > 64 && grid(128, 128) > 256) return launch_conv_runs<128, 128, 4, 2, 2, 1, 1>(p, s);
+            if (grid(128, 64) >= 256) return launch_conv_runs<128, 64, 2, 2, 2, 3, 1>(p, s);
+            return launch_conv_runs<64, 64, 2, 2, 3, 1, 1>(p, s);
+        }
         if (p.N <= 64) return launch_conv<128, 64, 2, 2, 2, 3>(p, s);
         // A round of 256 workgroups of 256x256 takes 1.85 of a round of 512 of
         // 128x128 (us, before -> after: 512^2 x 256 conv1 364 -> 337, conv2 391 ->
@@ -1109,24 +1125,30 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     //  143 x 3072 x 1024 9.8 -> 6.3 (32x64, 4 groups); 512 x 1152 x 1152 store
     //  10.7 -> 7.8, residual K = 2880 19.1 -> 15.3 (64x64, 2 groups).  From 1.3
     //  workgroups per CU on (324 64x64 tiles) the gain is 3 % and falls to none.
+    //  Where the rows that decide the order are fewer than the launch's (a batch
+    //  of images sums as one image does), k-groups stay while the launch's own
+    //  grid is that small; beyond it one group folds the runs on the tiles that
+    //  the grid fills (k-groups of 32x32 tiles there read four times the operand
+    //  bytes: 32 decodes of 8 x 8 latents 33.6 -> 29.2 ms, 8 of 16 x 16 29.6 -> 28.6).
     //  Sums that may not depend on M (the text encoder) take k_runs: 23 x 4096 x
     //  2304 15.2 -> 9.3, 23 x 2304 x 2304 15.2 -> 8.7; folding the same four runs
     //  in one group costs 738-row launches 0-2 %.  Its gate | up product keeps k
     //  in one sequence; up to 32 rows one-wave 32x32 tiles stream its weights at
     //  4.5 TB/s (27.0 -> 19.1 us).
-    if (p.k_runs == 4) {
-        if (grid(32, 32) <= 256) return launch_runs<32, 32, 1, 1, 3, 1, 4>(p, s);
-        if (p.M > 32 && p.M <= 64 && grid(64, 32) <= 256) return launch_runs<64, 32, 2, 1, 3, 1, 4>(p, s);
-        if (grid(32, 64) <= 256) return launch_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
-        if (grid(64, 64) <= 256) return launch_runs<64, 64, 2, 2, 2, 1, 4>(p, s);
-        if (grid(128, 128) > 256) return launch_runs<128, 128, 4, 2, 2, 1, 1>(p, s);
+    if (p.k_runs > 1) {
+        if (p.k_runs == 4) {
+            if (grid(32, 32) <= 256) return launch_runs<32, 32, 1, 1, 3, 1, 4>(p, s);
+            if (p.order_rows < 0 && p.M > 32 && p.M <= 64 && grid(64, 32) <= 256)
+                return launch_mode<64, 32, 2, 1, 3, kGemmStore, 1, kActNone, 0, 4>(
+                    p, ((p.M + 63) / 64) * ((p.N + 31) / 32), s);
+            if (grid(32, 64) <= (p.order_rows < 0 ? 256 : 288)) return launch_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
+            if (grid(64, 64) <= 256) return launch_runs<64, 64, 2, 2, 2, 1, 4>(p, s);
+        } else if (grid(64, 64) <= 256) {
+            return launch_runs<64, 64, 2, 2, 4, 1, 2>(p, s);
+        }
+        if (p.N > 64 && grid(128, 128) > 256) return launch_runs<128, 128, 4, 2, 2, 1, 1>(p, s);
         if (grid(128, 64) >= 256) return launch_runs<128, 64, 2, 2, 2, 3, 1>(p, s);
         return launch_runs<64, 64, 2, 2, 3, 1, 1>(p, s);
-    }
-    if (p.order_rows >= 0 && p.K >= 512 && p.batch == 1 && p.mode != kGemmVT && p.act != kActGeglu) {
-        if (grid(32, 32) <= 256) return launch_kg<32, 32, 1, 1, 3, 4>(p, s);
-        if (grid(32, 64) <= 288) return launch_kg<32, 64, 1, 2, 3, 4>(p, s);
-        if (grid(64, 64) <= 256) return launch_kg<64, 64, 2, 2, 4, 2>(p, s);
     }
     if (p.M <= 32 && p.mode == kGemmStore && p.N >= 8192) return launch<32, 32, 1, 1, 4, 1>(p, s);
     const int64_t tm128 = (p.M + 127) / 128;

@@ -94,6 +94,24 @@ def test_batch_matches_single():
         dev.close()
 
 
+# one image's products of 512 channels sum k in four runs at 4 x 4 pixels and in
+# two at 40 x 40; the batches take k-groups of 32x64 and 64x64 tiles, then one
+# group that folds the runs, on 64x64, 128x64 and 128x128 tiles
+@pytest.mark.parametrize("attn", [True, False], ids=["plain", "conv"])
+@pytest.mark.parametrize("side,batches", [(4, (2, 80, 130, 260, 520)), (40, (2, 3, 6))])
+def test_batches_sum_as_one_image(attn, side, batches):
+    ora, dev = build(dict(channels=(128, 512), attn=(False, attn)))
+    try:
+        lat = O.randn((batches[-1], 32, side, side), 17)
+        for b in batches:
+            whole = dev.decode(lat[:b])
+            assert np.isfinite(whole).all()
+            for i in sorted({0, b // 2, b - 1}):
+                assert np.array_equal(whole[i:i + 1], dev.decode(lat[i:i + 1])), (b, i)
+    finally:
+        dev.close()
+
+
 def test_256_tile_convs_equal_smaller_tiles():
     """The 3x3 convs of 182 x 202 pixels and 256 channels (plain, upsampling,
     conv_in) run on 256x256 tiles, those of the latent's upper part on 128x128
