@@ -151,7 +151,8 @@ int sana_dit_get_context(sana_dit * ctx, float * out);
 /* The forward of run_full_denoising_step_with_cfg (src/transformer.cpp:627-681):
  * latent [Bl, Cl, H, W] (repeated x2 for CFG), timestep t for every batch row,
  * the context set above (batch 2*Bl) -> noise_pred [2*Bl, Cl, H, W].  H * W
- * must be a perfect square (infer_square_side, src/transformer.cpp:18-24). */
+ * must be a perfect square (infer_square_side, src/transformer.cpp:18-24).  An
+ * image's prediction is the same, bit for bit, alone and in any batch. */
 int sana_dit_forward(sana_dit * ctx, const float * latent, int64_t Bl, int64_t H, int64_t W, float t,
                      float * noise_pred);
 /* Same with device pointers, asynchronous on `stream` (NULL = the context's stream). */

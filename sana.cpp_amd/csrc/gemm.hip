@@ -1051,7 +1051,8 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     if (p.k_runs == 1 && p.order_rows >= 0 &&
         (p.conv || (p.K >= 512 && p.batch == 1 && p.mode != kGemmVT && p.act != kActGeglu))) {
         const int64_t rows = p.order_rows > 0 ? p.order_rows : p.M;
-        auto order = [&](int bm, int bn) { return (rows + bm - 1) / bm * ((p.N + bn - 1) / bn) * co; };
+        const int64_t oco = p.order_co > 0 ? p.order_co : co;
+        auto order = [&](int bm, int bn) { return (rows + bm - 1) / bm * ((p.N + bn - 1) / bn) * oco; };
         if (order(32, 64) <= 288 || (!p.conv && order(32, 32) <= 256)) p.k_runs = 4;
         else if (order(64, 64) <= (p.conv ? 320 : 256)) p.k_runs = 2;
     }

@@ -81,11 +81,11 @@ struct GemmParams {
     int co = 1;
     // Order of the k sums.  order_rows: 0, small grids may sum k in parallel runs
     // chosen by the shape; > 0, the same with this many rows in place of M (a
-    // batch of images sums as one image does, on tiles chosen for the batch); < 0,
-    // k in one sequence whatever M is.  k_runs = 4 (plain stores): four runs of
+    // batch of images sums as one image does, on tiles chosen for the batch) and
+    // order_co (if > 0) in place of co; < 0, k in one sequence whatever M is.  k_runs = 4 (plain stores): four runs of
     // ceil(K / 64 / 4) k-tiles, each summed in sequence and added in order,
     // whatever M is.
-    int order_rows = 0, k_runs = 1;
+    int order_rows = 0, order_co = 0, k_runs = 1;
     int vec = 0;  // set by gemm(): 16-byte epilogue accesses are aligned
 };
 
