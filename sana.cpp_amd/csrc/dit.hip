@@ -120,6 +120,10 @@ struct sana_dit {
     // block chains as graphs, keyed by (chain, chains, batch rows, tokens, keys, masked);
     // they touch the context's own buffers only, so they are dropped where one is reallocated
     std::map<std::array<int64_t, 6>, hipGraphExec_t> graphs;
+    // recorded after the latest graph launches on their stream (which may be a
+    // caller's), so that no graph is destroyed while it may still run
+    hipEvent_t ev_graphs = nullptr;
+    bool graphs_queued = false;
     int64_t last_M = 0, last_B = 0, last_N = 0;
     int64_t loop_steps = 0, loop_n = 0;  // shape of the last denoise loop (its converted outputs stay in loop_x0)
     // Execution switches, read from the environment once by sana_dit_create:
@@ -128,6 +132,7 @@ struct sana_dit {
     bool cfg_branches = true, use_graphs = true;
 
     ~sana_dit() {
+        if (graphs_queued) (void)hipEventSynchronize(ev_graphs);
         for (auto & kv : graphs) (void)hipGraphExecDestroy(kv.second);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
@@ -135,6 +140,7 @@ struct sana_dit {
         if (ev_head_join) (void)hipEventDestroy(ev_head_join);
         if (ev_ctx) (void)hipEventDestroy(ev_ctx);
         if (ev_loop) (void)hipEventDestroy(ev_loop);
+        if (ev_graphs) (void)hipEventDestroy(ev_graphs);
         if (stream2) (void)hipStreamDestroy(stream2);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -143,6 +149,8 @@ struct sana_dit {
 namespace {
 
 void drop_graphs(sana_dit * c) {
+    if (c->graphs_queued) hip_check(hipEventSynchronize(c->ev_graphs), "graph cache");
+    c->graphs_queued = false;
     for (auto & kv : c->graphs) (void)hipGraphExecDestroy(kv.second);
     c->graphs.clear();
 }
@@ -621,24 +629,31 @@ hipGraphExec_t capture_graph(sana_dit * c, Body body) {
     return exec;
 }
 
-// Chain k of n over all blocks as a cached graph of its own.
-hipGraphExec_t chain_graph(sana_dit * c, int64_t k, int64_t n, int64_t B, int64_t N, const float * xbias) {
-    const std::array<int64_t, 6> key = {k, n, B, N, c->ctx_L, xbias != nullptr};
-    auto it = c->graphs.find(key);
-    if (it == c->graphs.end()) {
-        if (c->graphs.size() >= 64) {  // bounded: callers rarely use this many shapes
-            hip_check(hipStreamSynchronize(c->stream), "graph cache");
-            hip_check(hipStreamSynchronize(c->stream2), "graph cache");
-            drop_graphs(c);
+// The n chains over all blocks, each a cached graph of its own.
+constexpr size_t kMaxGraphs = 64;
+
+void chain_graphs(sana_dit * c, int64_t n, int64_t B, int64_t N, const float * xbias, hipGraphExec_t * out) {
+    auto key = [&](int64_t k) { return std::array<int64_t, 6>{k, n, B, N, c->ctx_L, xbias != nullptr}; };
+    size_t missing = 0;
+    for (int64_t k = 0; k < n; ++k) missing += !c->graphs.count(key(k));
+    // bounded (callers rarely use this many shapes); room is made before the first is fetched
+    if (missing && c->graphs.size() + missing > kMaxGraphs) drop_graphs(c);
+    const int64_t rows = B / n;
+    for (int64_t k = 0; k < n; ++k) {
+        hipGraphExec_t & e = c->graphs[key(k)];
+        if (!e) {
+            try {
+                e = capture_graph(c, [&](hipStream_t s) {
+                    for (int64_t i = 0; i < c->L_; ++i)
+                        enqueue_block(c, i, rows, N, xbias, s, nullptr, nullptr, k * rows, B, (int)n);
+                });
+            } catch (...) {
+                c->graphs.erase(key(k));
+                throw;
+            }
         }
-        const int64_t rows = B / n;
-        hipGraphExec_t e = capture_graph(c, [&](hipStream_t s) {
-            for (int64_t i = 0; i < c->L_; ++i)
-                enqueue_block(c, i, rows, N, xbias, s, nullptr, nullptr, k * rows, B, (int)n);
-        });
-        it = c->graphs.emplace(key, e).first;
+        out[k] = e;
     }
-    return it->second;
 }
 
 // Every block on x32, ordered on s.  Two chains are two linear graphs on two
@@ -651,27 +666,22 @@ hipGraphExec_t chain_graph(sana_dit * c, int64_t k, int64_t n, int64_t B, int64_
 // kernel of both by 1 us while its wait is queued.  xbias is the context's own
 // mask buffer or null.  `direct`: kernel launches instead of graphs.
 void run_all_blocks(sana_dit * c, int64_t B, int64_t N, const float * xbias, hipStream_t s, bool direct) {
-    const int64_t n = chain_count(c, B);
-    if (n == 1) {
-        if (direct)
-            for (int64_t i = 0; i < c->L_; ++i) enqueue_block(c, i, B, N, xbias, s);
-        else
-            hip_check(hipGraphLaunch(chain_graph(c, 0, 1, B, N, xbias), s), "hipGraphLaunch");
-        return;
-    }
+    const int64_t n = chain_count(c, B), rows = B / n;
     hipGraphExec_t g[2] = {nullptr, nullptr};
-    if (!direct)
-        for (int64_t k = 0; k < 2; ++k) g[k] = chain_graph(c, k, 2, B, N, xbias);
-    fork_to(c->ev_fork, s, c->stream2);
+    if (!direct) chain_graphs(c, n, B, N, xbias, g);
+    if (n == 2) fork_to(c->ev_fork, s, c->stream2);
     if (direct) {
         for (int64_t i = 0; i < c->L_; ++i)
-            for (int64_t k = 0; k < 2; ++k)
-                enqueue_block(c, i, B / 2, N, xbias, k ? c->stream2 : s, nullptr, nullptr, k * (B / 2), B, 2);
+            for (int64_t k = 0; k < n; ++k)
+                enqueue_block(c, i, rows, N, xbias, k ? c->stream2 : s, nullptr, nullptr, k * rows, B, (int)n);
     } else {
-        hip_check(hipGraphLaunch(g[0], s), "hipGraphLaunch");
-        hip_check(hipGraphLaunch(g[1], c->stream2), "hipGraphLaunch");
+        for (int64_t k = 0; k < n; ++k) hip_check(hipGraphLaunch(g[k], k ? c->stream2 : s), "hipGraphLaunch");
     }
-    join_from(c->ev_join, s, c->stream2);
+    if (n == 2) join_from(c->ev_join, s, c->stream2);
+    if (!direct) {
+        hip_check(hipEventRecord(c->ev_graphs, s), "hipEventRecord");
+        c->graphs_queued = true;
+    }
 }
 
 // The blocks and the final layer.
@@ -1035,6 +1045,7 @@ int sana_dit_create(const sana_dit_config * cfg, sana_dit ** out) {
         hip_check(hipEventCreateWithFlags(&c->ev_head_join, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipEventCreateWithFlags(&c->ev_ctx, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipEventCreateWithFlags(&c->ev_loop, hipEventDisableTiming), "hipEventCreate");
+        hip_check(hipEventCreateWithFlags(&c->ev_graphs, hipEventDisableTiming), "hipEventCreate");
         for (int64_t i = 0; i < c->L_; ++i) c->blocks.emplace_back(new BlockDev());
         // sinusoid frequencies exactly as the reference computes them in fp32
         // (src/transformer.cpp:89,97-99)

@@ -486,3 +486,41 @@ def test_small_step_streams_buffers_and_capture(small_model, images, masked):
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), ref)
         assert np.array_equal(step(data(71)), refs[1])
+
+
+def test_small_graph_cache_eviction(small_model, monkeypatch):
+    """More shapes than the graph cache holds (two chains each), queued on a
+    caller's stream without a wait: a graph is dropped only when it has run, and
+    every result equals direct launches."""
+    import sana_dit
+    import torch
+    m, _ = small_model
+    dev = torch.device("cuda:0")
+    cap = torch.from_numpy(O.randn((2, 16, 96), 91)).to(dev)
+    lat = torch.from_numpy(O.randn((1, 8, 8, 8), 92)).to(dev)
+    shapes = [(L, side, masked) for L in range(16, 0, -1) for side in (8, 7) for masked in (True, False)]
+    user = torch.cuda.Stream()
+
+    def run_all():
+        d = sana_dit.Dit(layers=2, hidden=128, ffn=256, caption_dim=96, latent_channels=8, self_heads=4, cross_heads=2)
+        try:
+            for name, shape in sana_dit.manifest(2, 128, 256, 96, 8).items():
+                d.set_weight(name, m.get(name, shape))
+            data = []
+            for L, side, masked in shapes:
+                bias = torch.zeros((2, L), device=dev)
+                bias[:, (L + 1) // 2:] = -10000.0
+                data.append((cap[:, :L].contiguous(), bias if masked else None, lat[:, :, :side, :side].contiguous(),
+                             torch.empty((2, 8, side, side), device=dev)))
+            torch.cuda.synchronize()
+            for (L, side, _), (c, b, x, out) in zip(shapes, data):
+                d.step_device(c, L, b, x, (1, 8, side, side), 999.0, out, user.cuda_stream)
+            torch.cuda.synchronize()
+            return [x[3].cpu().numpy() for x in data]
+        finally:
+            d.close()
+
+    got = run_all()
+    monkeypatch.setenv("SANA_DIT_NO_GRAPH", "1")
+    for shape, a, b in zip(shapes, got, run_all()):
+        assert np.isfinite(a).all() and np.array_equal(a, b), shape
