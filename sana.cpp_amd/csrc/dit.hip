@@ -88,7 +88,15 @@ void note_kernel(const char * name) { g_last_kernel = name; }
 const char * last_kernel() { return g_last_kernel; }
 }  // namespace sana
 
-struct sana_dit {
+// What a call leaves for later calls to check and read.
+struct DitState {
+    int64_t ctx_B = 0, ctx_L = 0, ctx_Lp = 0;  // conditioning
+    bool ctx_ready = false, ctx_bias = false;
+    int64_t last_M = 0, last_B = 0, last_N = 0;  // last forward
+    int64_t loop_steps = 0, loop_n = 0;  // last denoise loop (its converted outputs stay in loop_x0)
+};
+
+struct sana_dit : DitState {
     sana_dit_config cfg{};
     int64_t C = 0, E = 0, F = 0, Ccap = 0, Cl = 0, L_ = 0, Hs = 0, Hc = 0, Ds = 0, Dc = 0;
     int64_t Cp = 0, Fp = 0, Ccap_p = 0;  // K-padded row strides of GEMM operands
@@ -108,8 +116,6 @@ struct sana_dit {
     DevMem w_patch_t, b_patch, w_t1, b_t1, w_t2, b_t2, w_tp, b_tp, sst_final, w_proj, b_proj, freq;
     std::map<std::string, int> have;  // uploaded tensor names
     // context
-    int64_t ctx_B = 0, ctx_L = 0, ctx_Lp = 0;
-    bool ctx_ready = false, ctx_bias = false;
     DevMem cap32, cap16, caph16, capf32, ctx32, ctx16, kc, vt, bias;
     // forward workspace
     int64_t ws_M = 0, ws_B = 0;
@@ -124,8 +130,7 @@ struct sana_dit {
     // caller's), so that no graph is destroyed while it may still run
     hipEvent_t ev_graphs = nullptr;
     bool graphs_queued = false;
-    int64_t last_M = 0, last_B = 0, last_N = 0;
-    int64_t loop_steps = 0, loop_n = 0;  // shape of the last denoise loop (its converted outputs stay in loop_x0)
+    bool capturing = false;  // the current call's stream is being captured by the caller
     // Execution switches, read from the environment once by sana_dit_create:
     // SANA_DIT_CFG_BRANCHES=0 runs the CFG batch as one chain, SANA_DIT_NO_GRAPH=1
     // launches the blocks' kernels directly instead of replaying graphs.
@@ -354,7 +359,7 @@ void gemm_resid(const half_t * A, int64_t lda, const half_t * W, int64_t ldw, in
 void ensure_context_buffers(sana_dit * c, int64_t B, int64_t L) {
     const int64_t Lp = round_up(L, 32);
     if (B * L > c->ctx_B * c->ctx_L || Lp > c->ctx_Lp || B != c->ctx_B) {
-        drop_graphs(c);
+        if (!c->capturing) drop_graphs(c);  // (a capture's shape is undone after it)
         c->cap32.ensure((size_t)B * L * c->Ccap * 4);
         c->cap16.ensure((size_t)B * L * c->Ccap_p * 2);
         c->caph16.ensure((size_t)B * L * c->Cp * 2);
@@ -722,14 +727,29 @@ void enqueue_step(sana_dit * c, const float * caption, int64_t L, const float * 
     enqueue_body(c, Bl, N, xbias, out, s, direct);
 }
 
-// Whether work on s is launched kernel by kernel: with graphs off, and while
-// the caller captures s (it then becomes part of the caller's graph).
-bool direct_launches(const sana_dit * c, hipStream_t s) {
-    if (!c->use_graphs) return true;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (s != c->stream) hip_check(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing");
-    return cap != hipStreamCaptureStatusNone;
-}
+// A call on stream s.  While the caller captures s the kernels become part of the
+// caller's graph (kernel by kernel: direct_launches) and nothing runs, so the
+// state that later calls check and read is what it was before the call.
+class StreamCall {
+public:
+    StreamCall(sana_dit * c, hipStream_t s) : c_(c), before_(*c) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (s != c->stream) hip_check(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing");
+        c->capturing = cap != hipStreamCaptureStatusNone;
+    }
+    StreamCall(const StreamCall &) = delete;
+    StreamCall & operator=(const StreamCall &) = delete;
+    ~StreamCall() {
+        if (c_->capturing) static_cast<DitState &>(*c_) = before_;
+        c_->capturing = false;
+    }
+
+private:
+    sana_dit * c_;
+    DitState before_;
+};
+
+bool direct_launches(const sana_dit * c) { return !c->use_graphs || c->capturing; }
 
 // Tensors every block needs (load_block_weights, src/transformer.cpp:214-308).
 const char * const kBlockRequired[] = {
@@ -1456,6 +1476,7 @@ int sana_dit_forward_device(sana_dit * c, const float * d_latent, int64_t Bl, in
         return set_err(SANA_ERR_INVALID_ARGUMENT, "context batch size must equal 2 * latent batch size for CFG");
     return guarded([&] {
         hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
+        const StreamCall call(c, s);
         const int64_t B = 2 * Bl, N = Hh * Ww;
         ensure_forward_buffers(c, B, N);
         c->last_M = B * N;
@@ -1463,7 +1484,7 @@ int sana_dit_forward_device(sana_dit * c, const float * d_latent, int64_t Bl, in
         c->last_N = N;
         set_t(c, B, t, s);
         enqueue_forward(c, d_latent, Bl, N, c->ctx_bias ? c->bias.as<float>() : nullptr, d_out, s,
-                        direct_launches(c, s));
+                        direct_launches(c));
     });
 }
 
@@ -1495,6 +1516,7 @@ int sana_dit_step_device(sana_dit * c, const float * d_caption, int64_t L, const
     return guarded([&] {
         check_ready(c);
         hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
+        const StreamCall call(c, s);
         const int64_t B = 2 * Bl, N = Hh * Ww;
         ensure_context_buffers(c, B, L);
         ensure_forward_buffers(c, B, N);
@@ -1508,7 +1530,7 @@ int sana_dit_step_device(sana_dit * c, const float * d_caption, int64_t L, const
         if (d_bias)
             hip_check(hipMemcpyAsync(c->bias.p, d_bias, (size_t)B * L * 4, hipMemcpyDeviceToDevice, s), "bias");
         enqueue_step(c, d_caption, L, d_latent, Bl, N, d_bias ? c->bias.as<float>() : nullptr, d_out, s,
-                     direct_launches(c, s));
+                     direct_launches(c));
         c->ctx_ready = true;
     });
 }
@@ -1588,7 +1610,7 @@ float * enqueue_loop(sana_dit * c, const float * d_latent, int64_t Bl, int64_t H
     c->last_B = B;
     c->last_N = N;
     const float * xbias = c->ctx_bias ? c->bias.as<float>() : nullptr;
-    const bool direct = direct_launches(c, s);
+    const bool direct = direct_launches(c);
     hip_check(hipMemcpyAsync(c->loop_lat[0].p, d_latent, (size_t)n * 4, hipMemcpyDeviceToDevice, s), "latent");
     for (int64_t i = 0; i < steps; ++i) {
         float * cur = c->loop_lat[i & 1].as<float>();
@@ -1614,7 +1636,7 @@ float * enqueue_loop(sana_dit * c, const float * d_latent, int64_t Bl, int64_t H
                            first ? 0 : 1);
         hip_check(hipGetLastError(), "cfg_dpm");
     }
-    hip_check(hipEventRecord(c->ev_loop, s), "hipEventRecord");
+    if (!c->capturing) hip_check(hipEventRecord(c->ev_loop, s), "hipEventRecord");
     c->loop_steps = steps;
     c->loop_n = n;
     return c->loop_lat[steps & 1].as<float>();
@@ -1644,6 +1666,7 @@ int sana_dit_denoise_loop_device(sana_dit * c, const float * d_latent, int64_t B
     if (rc) return rc;
     return guarded([&] {
         hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
+        const StreamCall call(c, s);
         ensure_forward_buffers(c, 2 * Bl, Hh * Ww);
         float * res = enqueue_loop(c, d_latent, Bl, Hh, Ww, timesteps, sigmas, steps, guidance, s);
         hip_check(hipMemcpyAsync(d_final, res, (size_t)Bl * c->Cl * Hh * Ww * 4, hipMemcpyDeviceToDevice, s), "final");

@@ -524,3 +524,57 @@ def test_small_graph_cache_eviction(small_model, monkeypatch):
     monkeypatch.setenv("SANA_DIT_NO_GRAPH", "1")
     for shape, a, b in zip(shapes, got, run_all()):
         assert np.isfinite(a).all() and np.array_equal(a, b), shape
+
+
+def loop_outputs(d, shape):
+    import sana_dit
+    prev, last = np.empty(shape, np.float32), np.empty(shape, np.float32)
+    sana_dit.check(sana_dit.lib().sana_dit_loop_model_outputs(d.h, sana_dit.ptr(prev), sana_dit.ptr(last)))
+    return prev, last
+
+
+def test_small_capture_leaves_state(small_model):
+    """Recording a step (other caption length, masked) and a loop into a caller's
+    graphs runs nothing, so forwards and sana_dit_loop_model_outputs answer as
+    before; a step recorded after the conditioning was dropped does not bring it
+    back."""
+    import sana_dit
+    import torch
+    m, d = small_model
+    dev = torch.device("cuda:0")
+    latent, caption = O.randn((1, 8, 8, 8), 101), O.randn((2, 16, 96), 102)
+    ts6, sg6 = O.scheduler_timesteps(6)
+    ts4, sg4 = O.scheduler_timesteps(4)
+    d_lat = torch.from_numpy(latent).to(dev)
+    cap9 = torch.from_numpy(O.randn((2, 9, 96), 103)).to(dev)
+    bias9 = torch.zeros((2, 9), device=dev)
+    bias9[:, 4:] = -10000.0
+    out, fin = torch.empty((2, 8, 8, 8), device=dev), torch.empty((1, 8, 8, 8), device=dev)
+    d.set_context(caption, projected=False)
+    loop4 = d.denoise_loop(latent, ts4, sg4, 4.5)
+    d.denoise_loop(latent, ts6, sg6, 4.5)
+    x0 = loop_outputs(d, latent.shape)
+    ref = d.forward(latent, 999.0)
+    torch.cuda.synchronize()
+    user = torch.cuda.Stream()
+    step_graph, loop_graph = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(step_graph, stream=user):
+        d.step_device(cap9, 9, bias9, d_lat, (1, 8, 8, 8), 500.0, out, user.cuda_stream)
+    assert np.array_equal(d.forward(latent, 999.0), ref)
+    with torch.cuda.graph(loop_graph, stream=user):
+        d.denoise_loop_device(d_lat, (1, 8, 8, 8), ts4, sg4, 4.5, fin, user.cuda_stream)
+    for got, want in zip(loop_outputs(d, latent.shape), x0):
+        assert np.array_equal(got, want)
+    assert np.array_equal(d.forward(latent, 999.0), ref)
+    for _ in range(2):
+        fin.fill_(float("nan"))
+        loop_graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(fin.cpu().numpy(), loop4)
+        d.denoise_loop(latent, ts6, sg6, 4.5)
+    d.set_weight("caption_norm.weight", m.get("caption_norm.weight", (128,)))
+    with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=user):
+        d.step_device(cap9, 9, bias9, d_lat, (1, 8, 8, 8), 500.0, out, user.cuda_stream)
+    with pytest.raises(sana_dit.SanaError) as e:
+        d.forward(latent, 999.0)
+    assert e.value.code == sana_dit.SANA_ERR_STATE
