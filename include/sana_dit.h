@@ -16,6 +16,21 @@
  * stream, the device weights, a workspace and cached HIP graphs.  All device
  * memory is allocated by create / weight upload / the first call at a new
  * shape, never inside a captured graph.
+ *
+ * Capture: sana_dit_forward_device, sana_dit_step_device and
+ * sana_dit_denoise_loop_device on a stream that the caller captures become part
+ * of the caller's graph.
+ *  - Run the shape once before (growth during a capture is SANA_ERR_STATE).
+ *  - Recording runs nothing, so the context's state stays as it was: a recorded
+ *    step sets no conditioning, a recorded loop leaves nothing for
+ *    sana_dit_loop_model_outputs.
+ *  - The graph uses the context's buffers and weights and must not outlive it.
+ *    Later calls at larger shapes are fine: outgrown buffers then stay allocated
+ *    until sana_dit_destroy.
+ *  - A replay overwrites the buffers as the call would (a step the conditioning,
+ *    a loop the kept outputs), without the context knowing: order replays with
+ *    the context's other work, and set the conditioning again before a forward
+ *    or a loop that follows a replayed step.
  */
 #ifndef SANA_DIT_H
 #define SANA_DIT_H

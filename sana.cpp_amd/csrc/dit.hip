@@ -131,6 +131,10 @@ struct sana_dit : DitState {
     hipEvent_t ev_graphs = nullptr;
     bool graphs_queued = false;
     bool capturing = false;  // the current call's stream is being captured by the caller
+    // a caller's graph may hold the buffers (a call was captured): those outgrown
+    // since then are kept until the context goes
+    bool captured = false;
+    std::vector<void *> retired;
     // Execution switches, read from the environment once by sana_dit_create:
     // SANA_DIT_CFG_BRANCHES=0 runs the CFG batch as one chain, SANA_DIT_NO_GRAPH=1
     // launches the blocks' kernels directly instead of replaying graphs.
@@ -139,6 +143,7 @@ struct sana_dit : DitState {
     ~sana_dit() {
         if (graphs_queued) (void)hipEventSynchronize(ev_graphs);
         for (auto & kv : graphs) (void)hipGraphExecDestroy(kv.second);
+        for (void * p : retired) (void)hipFree(p);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
         if (ev_head_fork) (void)hipEventDestroy(ev_head_fork);
@@ -356,19 +361,33 @@ void gemm_resid(const half_t * A, int64_t lda, const half_t * W, int64_t ldw, in
     launch_check(sana::gemm(p, s), "gemm_residual");
 }
 
+// A context buffer of at least n bytes.  Nothing is allocated (or freed) while
+// the caller captures.
+void grow(sana_dit * c, DevMem & m, size_t n, bool zero = true) {
+    if (n <= m.bytes && m.p) return;
+    if (c->capturing)
+        throw_err(SANA_ERR_STATE, "a captured call cannot allocate: run its shape once before the capture");
+    if (c->captured && m.p) {
+        c->retired.push_back(m.p);
+        m.p = nullptr;
+        m.bytes = 0;
+    }
+    m.ensure(n, zero);
+}
+
 void ensure_context_buffers(sana_dit * c, int64_t B, int64_t L) {
     const int64_t Lp = round_up(L, 32);
     if (B * L > c->ctx_B * c->ctx_L || Lp > c->ctx_Lp || B != c->ctx_B) {
         if (!c->capturing) drop_graphs(c);  // (a capture's shape is undone after it)
-        c->cap32.ensure((size_t)B * L * c->Ccap * 4);
-        c->cap16.ensure((size_t)B * L * c->Ccap_p * 2);
-        c->caph16.ensure((size_t)B * L * c->Cp * 2);
-        c->capf32.ensure((size_t)B * L * c->C * 4);
-        c->ctx32.ensure((size_t)B * L * c->C * 4);
-        c->ctx16.ensure((size_t)B * L * c->Cp * 2);
-        c->kc.ensure((size_t)B * L * c->L_ * c->C * 2);
-        c->vt.ensure((size_t)c->L_ * B * c->C * Lp * 2);  // zero: key padding must read as 0
-        c->bias.ensure((size_t)B * L * 4);
+        grow(c, c->cap32, (size_t)B * L * c->Ccap * 4);
+        grow(c, c->cap16, (size_t)B * L * c->Ccap_p * 2);
+        grow(c, c->caph16, (size_t)B * L * c->Cp * 2);
+        grow(c, c->capf32, (size_t)B * L * c->C * 4);
+        grow(c, c->ctx32, (size_t)B * L * c->C * 4);
+        grow(c, c->ctx16, (size_t)B * L * c->Cp * 2);
+        grow(c, c->kc, (size_t)B * L * c->L_ * c->C * 2);
+        grow(c, c->vt, (size_t)c->L_ * B * c->C * Lp * 2);  // zero: key padding must read as 0
+        grow(c, c->bias, (size_t)B * L * 4);
         c->ctx_Lp = Lp;
     }
     c->ctx_B = B;
@@ -430,29 +449,29 @@ void enqueue_context(sana_dit * c, const float * caption, bool projected, int64_
 void ensure_forward_buffers(sana_dit * c, int64_t B, int64_t N) {
     const int64_t M = B * N;
     if (M > c->ws_M || B > c->ws_B) {
-        drop_graphs(c);
+        if (!c->capturing) drop_graphs(c);
         const int64_t C = c->C;
-        c->x32.ensure((size_t)M * C * 4);
-        c->fin32.ensure((size_t)M * C * 4);
-        c->xa16.ensure((size_t)M * c->Cp * 2);
-        c->qkv16.ensure((size_t)M * 3 * C * 2);
-        c->la_kt.ensure((size_t)M * C * 2);
-        c->la_vt.ensure((size_t)M * C * 2);
-        c->o16.ensure((size_t)M * c->Cp * 2);
-        c->r16.ensure((size_t)M * c->Cp * 2);
-        c->q16.ensure((size_t)M * C * 2);
-        c->hid16.ensure((size_t)M * c->E * 2);
-        c->glu16.ensure((size_t)M * c->Fp * 2);
+        grow(c, c->x32, (size_t)M * C * 4);
+        grow(c, c->fin32, (size_t)M * C * 4);
+        grow(c, c->xa16, (size_t)M * c->Cp * 2);
+        grow(c, c->qkv16, (size_t)M * 3 * C * 2);
+        grow(c, c->la_kt, (size_t)M * C * 2);
+        grow(c, c->la_vt, (size_t)M * C * 2);
+        grow(c, c->o16, (size_t)M * c->Cp * 2);
+        grow(c, c->r16, (size_t)M * c->Cp * 2);
+        grow(c, c->q16, (size_t)M * C * 2);
+        grow(c, c->hid16, (size_t)M * c->E * 2);
+        grow(c, c->glu16, (size_t)M * c->Fp * 2);
         // for any token count: a later call of fewer tokens may split them into more chunks
-        c->la_ws.ensure(sana::linattn_workspace_floats_any((int)B, (int)c->Hs, (int)c->Ds) * 4);
-        c->la_ws2.ensure(sana::linattn_workspace_floats_any((int)((B + 1) / 2), (int)c->Hs, (int)c->Ds) * 4);
-        c->d_t.ensure((size_t)B * 4);
-        c->e1.ensure((size_t)B * C * 4);
-        c->emb.ensure((size_t)B * C * 4);
-        c->tmod.ensure((size_t)B * 6 * C * 4);
-        c->mod_all.ensure((size_t)c->L_ * B * 6 * C * 4);
-        c->lat_in.ensure((size_t)B * c->Cl * N * 4);
-        c->np_out.ensure((size_t)B * c->Cl * N * 4);
+        grow(c, c->la_ws, sana::linattn_workspace_floats_any((int)B, (int)c->Hs, (int)c->Ds) * 4);
+        grow(c, c->la_ws2, sana::linattn_workspace_floats_any((int)((B + 1) / 2), (int)c->Hs, (int)c->Ds) * 4);
+        grow(c, c->d_t, (size_t)B * 4);
+        grow(c, c->e1, (size_t)B * C * 4);
+        grow(c, c->emb, (size_t)B * C * 4);
+        grow(c, c->tmod, (size_t)B * 6 * C * 4);
+        grow(c, c->mod_all, (size_t)c->L_ * B * 6 * C * 4);
+        grow(c, c->lat_in, (size_t)B * c->Cl * N * 4);
+        grow(c, c->np_out, (size_t)B * c->Cl * N * 4);
         c->ws_M = M;
         c->ws_B = B;
     }
@@ -736,6 +755,7 @@ public:
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (s != c->stream) hip_check(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing");
         c->capturing = cap != hipStreamCaptureStatusNone;
+        c->captured = c->captured || c->capturing;
     }
     StreamCall(const StreamCall &) = delete;
     StreamCall & operator=(const StreamCall &) = delete;
@@ -1603,8 +1623,8 @@ float * enqueue_loop(sana_dit * c, const float * d_latent, int64_t Bl, int64_t H
     const int64_t n = Bl * c->Cl * Hh * Ww;
     const int64_t B = 2 * Bl, N = Hh * Ww;
     for (int k = 0; k < 2; ++k) {
-        c->loop_lat[k].ensure((size_t)n * 4, false);
-        c->loop_x0[k].ensure((size_t)n * 4, false);
+        grow(c, c->loop_lat[k], (size_t)n * 4, false);
+        grow(c, c->loop_x0[k], (size_t)n * 4, false);
     }
     c->last_M = B * N;
     c->last_B = B;

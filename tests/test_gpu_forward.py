@@ -578,3 +578,59 @@ def test_small_capture_leaves_state(small_model):
     with pytest.raises(sana_dit.SanaError) as e:
         d.forward(latent, 999.0)
     assert e.value.code == sana_dit.SANA_ERR_STATE
+
+
+def test_small_growth_after_capture(small_model):
+    """A captured step replays correctly after larger eager calls have outgrown
+    the buffers it holds (context and workspace), and a capture of a shape that
+    was never run is refused with everything as before."""
+    import sana_dit
+    import torch
+    m, _ = small_model
+    dev = torch.device("cuda:0")
+    d = sana_dit.Dit(layers=2, hidden=128, ffn=256, caption_dim=96, latent_channels=8, self_heads=4, cross_heads=2)
+    user = torch.cuda.Stream()
+
+    def data(images, side, L, seed):
+        return (torch.from_numpy(O.randn((2 * images, L, 96), seed)).to(dev),
+                torch.from_numpy(O.randn((images, 8, side, side), seed + 1)).to(dev),
+                torch.full((2 * images, 8, side, side), float("nan"), device=dev))
+
+    def step(x):
+        torch.cuda.synchronize()
+        d.step_device(x[0], x[0].shape[1], None, x[1], tuple(x[1].shape), 999.0, x[2], user.cuda_stream)
+
+    def eager(*a):
+        x = data(*a)
+        step(x)
+        torch.cuda.synchronize()
+        return x[2].cpu().numpy()
+
+    try:
+        for name, shape in sana_dit.manifest(2, 128, 256, 96, 8).items():
+            d.set_weight(name, m.get(name, shape))
+        ref = eager(1, 8, 16, 111)
+        x = data(1, 8, 16, 111)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=user):
+            d.step_device(x[0], 16, None, x[1], (1, 8, 8, 8), 999.0, x[2], user.cuda_stream)
+        large = data(2, 16, 40, 121)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=user):
+            with pytest.raises(sana_dit.SanaError) as e:
+                d.step_device(large[0], 40, None, large[1], (2, 8, 16, 16), 999.0, large[2], user.cuda_stream)
+        assert e.value.code == sana_dit.SANA_ERR_STATE
+        assert np.array_equal(eager(1, 8, 16, 111), ref)
+        want = eager(2, 16, 40, 121)
+        for _ in range(3):
+            x[2].fill_(float("nan"))
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(x[2].cpu().numpy(), ref)
+            assert np.array_equal(eager(2, 16, 40, 121), want)
+        del g
+        torch.cuda.synchronize()
+    finally:
+        d.close()
