@@ -378,7 +378,12 @@ void grow(sana_dit * c, DevMem & m, size_t n, bool zero = true) {
 void ensure_context_buffers(sana_dit * c, int64_t B, int64_t L) {
     const int64_t Lp = round_up(L, 32);
     if (B * L > c->ctx_B * c->ctx_L || Lp > c->ctx_Lp || B != c->ctx_B) {
-        if (!c->capturing) drop_graphs(c);  // (a capture's shape is undone after it)
+        if (!c->capturing) {  // (a capture's shape is undone after it)
+            drop_graphs(c);
+            // no shape and no conditioning until every buffer is there
+            c->ctx_B = c->ctx_L = c->ctx_Lp = 0;
+            c->ctx_ready = false;
+        }
         grow(c, c->cap32, (size_t)B * L * c->Ccap * 4);
         grow(c, c->cap16, (size_t)B * L * c->Ccap_p * 2);
         grow(c, c->caph16, (size_t)B * L * c->Cp * 2);
@@ -449,7 +454,10 @@ void enqueue_context(sana_dit * c, const float * caption, bool projected, int64_
 void ensure_forward_buffers(sana_dit * c, int64_t B, int64_t N) {
     const int64_t M = B * N;
     if (M > c->ws_M || B > c->ws_B) {
-        if (!c->capturing) drop_graphs(c);
+        if (!c->capturing) {
+            drop_graphs(c);
+            c->ws_M = c->ws_B = 0;  // until every buffer is there
+        }
         const int64_t C = c->C;
         grow(c, c->x32, (size_t)M * C * 4);
         grow(c, c->fin32, (size_t)M * C * 4);

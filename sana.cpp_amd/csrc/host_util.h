@@ -125,7 +125,12 @@ struct DevMem {
         if (p) hip_check(hipFree(p), "hipFree");
         p = nullptr;
         bytes = 0;
-        hip_check(hipMalloc(&p, n ? n : 16), "hipMalloc");
+        const hipError_t e = hipMalloc(&p, n ? n : 16);
+        if (e != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();  // reported here, not by the next launch's check
+        }
+        hip_check(e, "hipMalloc");
         bytes = n;
         if (zero) {
             // A device memset may return before it completes, and work on a

@@ -634,3 +634,38 @@ def test_small_growth_after_capture(small_model):
         torch.cuda.synchronize()
     finally:
         d.close()
+
+
+def test_small_step_after_failed_growth():
+    """A step whose workspace does not fit the device fails with
+    SANA_ERR_OUT_OF_MEMORY; the context then allocates what the next shape needs
+    instead of running on the buffers that were given up."""
+    import sana_dit
+    import torch
+    dev = torch.device("cuda:0")
+    m = O.Model(**SMALL)
+    d = sana_dit.Dit(layers=2, hidden=128, ffn=256, caption_dim=96, latent_channels=8, self_heads=4, cross_heads=2)
+    try:
+        for name, shape in sana_dit.manifest(2, 128, 256, 96, 8).items():
+            d.set_weight(name, m.get(name, shape))
+        cap = torch.from_numpy(O.randn((2, 16, 96), 131)).to(dev)
+        lat = torch.from_numpy(O.randn((1, 8, 8, 8), 132)).to(dev)
+        out = torch.empty((2, 8, 8, 8), device=dev)
+
+        def step():
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            d.step_device(cap, 16, None, lat, (1, 8, 8, 8), 999.0, out)
+            torch.cuda.synchronize()
+            return out.cpu().numpy()
+
+        ref = step()
+        with pytest.raises(sana_dit.SanaError) as e:  # 1.3 TB for the residual stream alone
+            d.step_device(cap, 1, None, lat, (20000, 8, 255, 255), 999.0, out)
+        assert e.value.code == sana_dit.SANA_ERR_OUT_OF_MEMORY
+        with pytest.raises(sana_dit.SanaError) as e:
+            d.forward_device(lat, (1, 8, 8, 8), 999.0, out)
+        assert e.value.code == sana_dit.SANA_ERR_STATE
+        assert np.array_equal(step(), ref)
+    finally:
+        d.close()
