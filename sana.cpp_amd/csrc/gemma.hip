@@ -35,6 +35,7 @@
 #include "hip_common.h"
 #include "host_util.h"
 #include "kernels.h"
+#include "soft_math.h"
 
 using sana::half_t;
 using namespace sana_host;
@@ -242,22 +243,6 @@ __global__ __launch_bounds__(256) void gemma_qkv_kernel(const float * __restrict
     }
 }
 
-// e^x for x <= 0 (0 for -inf, NaN for NaN) on v_exp_f32: the exponent's rounding
-// leaves a relative error of |x| 2^-24 on top of the instruction's 1 ulp, far
-// below the fp16 rounding of the probabilities.
-__device__ inline float exp_f32(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
-
-// tanh to a few ulp: below 1/4 its series to x^9 (the next term is 9e-9 of it),
-// above 1 - 2 / (e^2x + 1).  Against expf and tanhf, whose branches every lane
-// walks: attention of 438 + 300 tokens 27.1 -> 25.0 us, of 23 tokens 10.4 -> 8.0.
-__device__ inline float tanh_f32(float x) {
-    const float t = x * x;
-    const float poly = x + x * t * (-1.0f / 3 + t * (2.0f / 15 + t * (-17.0f / 315 + t * (62.0f / 2835))));
-    const float a = fabsf(x);
-    const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a * 2.88539008f) + 1.0f);
-    return a < 0.25f ? poly : copysignf(big, x);
-}
-
 // Causal soft-capped attention with a sliding window, one pass (online
 // softmax), for all sequences and heads in one launch: head dims D of 64, 128
 // and 256 (others take attention_by_products: the score product, the softmax
@@ -271,11 +256,13 @@ __device__ inline float tanh_f32(float x) {
 // its K block (32 x D) and V^T block (D x 32) in LDS of its own by direct
 // global -> LDS DMA, whole rows at a time (fragments read straight from global
 // memory touch 32 lines per instruction: 30 us for 438 + 300 tokens against
-// 25; 23 tokens 8.0 us).  The next block's K is requested when this one's
+// 23.9; 23 tokens 8.3 us).  The next block's K is requested when this one's
 // fragments are in registers, its V^T when this one's products are done.  What
 // bounds it is the chain of one wave's key blocks (up to 4 here): the
 // accumulators, q and K take the registers of one wave per SIMD, so nothing
-// hides a block's LDS reads and exponentials.
+// hides a block's LDS reads and exponentials.  These keep the accuracy of expf and
+// tanhf (soft_math.h) and of a division by the cap; while every |score| of a wave's
+// block is below the cap, tanh is its polynomial alone.
 // S^T = K Q^T (K rows as the first MFMA operand, q in registers), so a lane
 // holds 16 keys of one query, exactly what it feeds back as the P^T operand of
 // O^T = V^T P^T: the contraction takes key 16 s + 8 (e / 4) + 4 (lane / 32) + e %
@@ -361,23 +348,39 @@ __global__ __launch_bounds__(256, 1) void gemma_attention_kernel(const f16 * __r
             sd = mfma_32x32x16(kf[s + 1], qf[s + 1], sd);
         }
         // lane: query q0 + ql, keys k0 + 8 (e / 4) + 4 hf + e % 4
+        float um = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            // score / cap to its last bit: a quotient by the rounded 1 / cap (far past
+            // tanh's range cut off, so that no inf - inf arises) and its correction
+            const float x = sc[e] + sd[e], u = __builtin_amdgcn_fmed3f(x * inv_cap, -64.0f, 64.0f);
+            sc[e] = fmaf(fmaf(-u, cap, x), inv_cap, u);
+            um = fmaxf(um, fabsf(sc[e]));
+        }
+        if (__any(um >= 1.0f)) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sc[e] = cap * sana::soft_tanh(sc[e]);
+        } else {  // the same without the other branch of tanh
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sc[e] = cap * sana::soft_tanh_below_1(sc[e]);
+        }
         float bm = -INFINITY;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int j = k0 + 8 * (e >> 2) + 4 * hf + (e & 3), t = q0 + ql;
             const bool in = j <= t && j < T && (window <= 0 || j > t - window);
-            sc[e] = in ? cap * tanh_f32((sc[e] + sd[e]) * inv_cap) : -INFINITY;
+            sc[e] = in ? sc[e] : -INFINITY;
             bm = fmaxf(bm, sc[e]);
         }
         bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
         const float mn = fmaxf(mx, bm);
         // a query without a key so far keeps sums of zero
-        const float f = mx == -INFINITY ? 0.0f : exp_f32(mx - mn);
+        const float m0 = mn == -INFINITY ? 0.0f : mn, f = expf(mx - m0);
         float bs = 0.0f;
         f16x8 pf[2];
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const float p = sc[e] == -INFINITY ? 0.0f : exp_f32(sc[e] - mn);
+            const float p = expf(sc[e] - m0);
             bs += p;
             pf[e >> 3][e & 7] = (f16)p;
         }
@@ -435,10 +438,10 @@ __global__ __launch_bounds__(256, 1) void gemma_attention_kernel(const f16 * __r
     for (int v = 0; v < nw; ++v) gm = fmaxf(gm, stat[v * 64 + ql]);
     for (int v = 0; v < nw; ++v) {
         const float m = stat[v * 64 + ql];
-        gs += m == -INFINITY ? 0.0f : stat[v * 64 + 32 + ql] * exp_f32(m - gm);
+        gs += m == -INFINITY ? 0.0f : stat[v * 64 + 32 + ql] * expf(m - gm);
     }
     if (w < nw) {
-        const float f = mx == -INFINITY ? 0.0f : exp_f32(mx - gm);
+        const float f = mx == -INFINITY ? 0.0f : expf(mx - gm);
 #pragma unroll
         for (int j = 0; j < DT; ++j)
 #pragma unroll
@@ -675,8 +678,10 @@ std::vector<Seq> layout(const sana_gemma * g, const std::vector<int64_t> & lens)
 }
 
 bool one_pass_attention(const sana_gemma_config & c) {
-    // (32-bit offsets into the K rows: up to 8192 tokens)
-    return (c.head_dim == 64 || c.head_dim == 128 || c.head_dim == 256) && c.kv_heads * c.head_dim <= 65536;
+    // (32-bit offsets into the K rows: up to 8192 tokens; a soft cap whose
+    // reciprocal and quotients are normal numbers)
+    return (c.head_dim == 64 || c.head_dim == 128 || c.head_dim == 256) && c.kv_heads * c.head_dim <= 65536 &&
+           c.attn_softcap >= 1e-20f && c.attn_softcap <= 1e20f;
 }
 
 void ensure_workspace(sana_gemma * g, const std::vector<Seq> & q) {

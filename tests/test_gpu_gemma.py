@@ -194,3 +194,17 @@ def test_norm_widths_vs_oracle(hidden, ffn):
         assert rel_l2(dev.encode(tokens), G.forward(w, cfg, tokens)) < TOL
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("d", [64, 256])
+@pytest.mark.parametrize("cap", [0.02, 0.7, 1e19, 1e25])
+def test_softcap_ranges_vs_oracle(d, cap):
+    """Scores far past the soft cap, around it (both branches of tanh) and far below
+    it; the last cap takes the product path."""
+    cfg = dict(EDGE, head_dim=d, softcap=cap, query_scale=d ** -0.5)
+    w, dev = build(cfg, scale=0.1)
+    try:
+        tokens = np.random.default_rng(d).integers(0, cfg["vocab"], size=97)
+        assert rel_l2(dev.encode(tokens), G.forward(w, cfg, tokens)) < TOL
+    finally:
+        dev.close()
