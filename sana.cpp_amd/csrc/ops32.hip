@@ -722,7 +722,7 @@ int sana_op_gemm_f32(const float * A, int64_t lda, int64_t strideA, const float 
     for (int i = 0; i < 3; ++i) {
         const int64_t t = ((M + tiles[i].m - 1) / tiles[i].m) * ((N + tiles[i].n - 1) / tiles[i].n) * batch;
         const int64_t cost = tiles[i].fixed + (t + 255) / 256 * tiles[i].round;
-        if (t / batch <= INT32_MAX && cost < best_cost) {
+        if (t / batch < (1 << 24) && cost < best_cost) {  // a launch holds fewer than 2^32 threads per axis
             best = i;
             best_cost = cost;
         }

@@ -133,3 +133,15 @@ def test_heads_f32(L, B, N, H, D, off):
     L.check(L.lib().sana_op_heads_f32(y.data_ptr(), z.data_ptr(), B, N, H, D, 0, None))
     assert np.array_equal(down(y, (B, H, N, D)), x.transpose(0, 2, 1, 3))
     assert np.array_equal(down(z, (B, N, H, D)), x)
+
+
+def test_gemm_f32_widest_row(L):
+    """2^29 columns and more: 32-column tiles would need 2^32 threads in a launch."""
+    n = (1 << 29) + 37
+    a = torch.full((1,), 1.5, device="cuda")
+    b = torch.arange(n, device="cuda", dtype=torch.float32)
+    c = torch.full((n,), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    L.check(L.lib().sana_op_gemm_f32(a.data_ptr(), 1, 0, b.data_ptr(), n, 0, 0, None, 1, c.data_ptr(), n, 0, 1, n, 1,
+                                     1, 0, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(c, b.mul_(1.5))
