@@ -1045,6 +1045,9 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     if (p.bias) vec = vec && (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0;
     p.vec = vec ? 1 : 0;
     const int64_t co = std::max(p.co, 1) * (int64_t)p.batch;
+    // 32x64 tiles with four k-groups, one workgroup per CU: a few more than 256 still
+    // fit a round where another launch shares the CUs, alone they take a second one
+    auto one_round = [](int64_t launches) { return launches > 1 ? 288 : 256; };
     auto grid = [&](int bm, int bn) { return ((int64_t)p.M + bm - 1) / bm * ((p.N + bn - 1) / bn) * co; };
     // The order of the k sums follows from the rows that decide it alone
     // (GemmParams::order_rows), the tiles below from the launch's own rows.
@@ -1053,7 +1056,7 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
         const int64_t rows = p.order_rows > 0 ? p.order_rows : p.M;
         const int64_t oco = p.order_co > 0 ? p.order_co : co;
         auto order = [&](int bm, int bn) { return (rows + bm - 1) / bm * ((p.N + bn - 1) / bn) * oco; };
-        if (order(32, 64) <= 288 || (!p.conv && order(32, 32) <= 256)) p.k_runs = 4;
+        if (order(32, 64) <= one_round(oco) || (!p.conv && order(32, 32) <= 256)) p.k_runs = 4;
         else if (order(64, 64) <= (p.conv ? 320 : 256)) p.k_runs = 2;
     }
     // Rounds (in 1/64) of `slots` workgroups at a time that bm x bn tiles of all
@@ -1063,7 +1066,7 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
         return co > 1 ? std::max<int64_t>(64, t * 64 / slots) : (t + slots - 1) / slots * 64;
     };
     if (p.conv) {
-        if (p.k_runs == 4 && grid(32, 64) <= 288) return launch_conv_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
+        if (p.k_runs == 4 && grid(32, 64) <= one_round(co)) return launch_conv_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
         if (p.k_runs == 4 && grid(64, 64) <= 256) return launch_conv_runs<64, 64, 2, 2, 2, 1, 4>(p, s);
         if (p.k_runs == 2 && grid(64, 64) <= 320) return launch_conv_runs<64, 64, 2, 2, 4, 1, 2>(p, s);
         if (p.k_runs > 1) {
@@ -1124,7 +1127,10 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     // workgroup per CU; graph chains, us per launch, before -> after (M x N x K):
     //  128 x 1152 x 1152 residual 11.5 -> 6.4, K = 2880 18.3 -> 9.6 (32x32, 4 groups);
     //  143 x 3072 x 1024 9.8 -> 6.3 (32x64, 4 groups); 512 x 1152 x 1152 store
-    //  10.7 -> 7.8, residual K = 2880 19.1 -> 15.3 (64x64, 2 groups).  From 1.3
+    //  10.7 -> 7.8, residual K = 2880 19.1 -> 15.3 (64x64, 2 groups).  32x64 tiles
+    //  stay to 288 of them only beside another launch: alone those are a second
+    //  round (33 x 9000 x 1024, 282 of them 10.0 us with weights in the cache and
+    //  11.8 without, 141 of 64x64 in 2 groups 6.9 and 7.8).  From 1.3
     //  workgroups per CU on (324 64x64 tiles) the gain is 3 % and falls to none.
     //  Where the rows that decide the order are fewer than the launch's (a batch
     //  of images sums as one image does), k-groups stay while the launch's own
@@ -1134,15 +1140,16 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     //  Sums that may not depend on M (the text encoder) take k_runs: 23 x 4096 x
     //  2304 15.2 -> 9.3, 23 x 2304 x 2304 15.2 -> 8.7; folding the same four runs
     //  in one group costs 738-row launches 0-2 %.  Its gate | up product keeps k
-    //  in one sequence; up to 32 rows one-wave 32x32 tiles stream its weights at
-    //  4.5 TB/s (27.0 -> 19.1 us).
+    //  in one sequence; up to 32 rows one-wave 32x32 tiles stream its weights from
+    //  memory at 4.5 TB/s (27.0 -> 19.1 us; only there: a plain store whose weights
+    //  are in the cache is slower on them, 32 x 18432 x 2304 18.9 -> 21.3).
     if (p.k_runs > 1) {
         if (p.k_runs == 4) {
             if (grid(32, 32) <= 256) return launch_runs<32, 32, 1, 1, 3, 1, 4>(p, s);
             if (p.order_rows < 0 && p.M > 32 && p.M <= 64 && grid(64, 32) <= 256)
                 return launch_mode<64, 32, 2, 1, 3, kGemmStore, 1, kActNone, 0, 4>(
                     p, ((p.M + 63) / 64) * ((p.N + 31) / 32), s);
-            if (grid(32, 64) <= (p.order_rows < 0 ? 256 : 288)) return launch_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
+            if (grid(32, 64) <= (p.order_rows < 0 ? 256 : one_round(co))) return launch_runs<32, 64, 1, 2, 3, 1, 4>(p, s);
             if (grid(64, 64) <= 256) return launch_runs<64, 64, 2, 2, 2, 1, 4>(p, s);
         } else if (grid(64, 64) <= 256) {
             return launch_runs<64, 64, 2, 2, 4, 1, 2>(p, s);
@@ -1151,7 +1158,7 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
         if (grid(128, 64) >= 256) return launch_runs<128, 64, 2, 2, 2, 3, 1>(p, s);
         return launch_runs<64, 64, 2, 2, 3, 1, 1>(p, s);
     }
-    if (p.M <= 32 && p.mode == kGemmStore && p.N >= 8192) return launch<32, 32, 1, 1, 4, 1>(p, s);
+    if (p.M <= 32 && p.act == kActGeglu && p.N >= 8192) return launch<32, 32, 1, 1, 4, 1>(p, s);
     const int64_t tm128 = (p.M + 127) / 128;
     const int64_t t128 = tm128 * ((p.N + 127) / 128) * co;
     if (t128 <= 160) {
