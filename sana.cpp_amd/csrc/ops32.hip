@@ -34,7 +34,7 @@ struct OpGemm {
     const float * bias;
     float * C;
     int64_t lda, ldb, ldc, sA, sB, sC;
-    int M, N, K, bias_mode, accumulate, vec_c;
+    int M, N, K, bias_mode, accumulate;
 };
 
 constexpr int kTK = 32;
@@ -52,18 +52,21 @@ constexpr int kTK = 32;
 // (conflict-free 16-byte reads of 16 rows); a lane's 16 bytes feed four MFMAs,
 // so product j of a 16-deep step contracts k = 16 s + 4 g + j over the lane
 // groups g.  B [K, N] lies as rows of BN + 4 floats, read four k rows apart
-// (64 distinct banks).  The MFMA computes the transposed tile, so a lane
-// stores four consecutive columns.
+// (64 distinct banks).
 //
 // VA, VB: floats per global load of A and B, 4 where base, strides and extents
-// are multiples of 4 elements (16 bytes), else 1.
+// are multiples of 4 elements (16 bytes), else 1.  VC, where the same holds for
+// C's base and strides: the MFMA computes the transposed tile and a lane stores
+// four consecutive columns of a row at once; else the tile itself, and a store
+// covers 16 consecutive columns of four rows (16 products of 1023 x 1021 x 64 50.2 ->
+// 34.8 us; as single elements of the transposed tile those were 16 bytes apart).
 //
 // Measured on MI355X: 2048 x 1152 x 1152 65 us (84 TFLOP/s); with the other
 // kernels of this file the fp32 self-attention block (2 x 1024 tokens, four
 // such products) went from 1316 to 288 us and the cross-attention block (2 x
 // 256 tokens, 300 keys) from 787 to 139 us, against a 64 x 64 tile with
 // single-buffered 16-deep k-tiles and two barriers each.
-template <int BM, int BN, bool BT, int VA, int VB>
+template <int BM, int BN, bool BT, int VA, int VB, bool VC>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(OpGemm p, int tiles_n) {
     constexpr int TM = BM / 32, TN = BN / 32;        // 16 x 16 tiles per wave
     constexpr int AF = BM * kTK / 256, BF = BN * kTK / 256;  // floats per thread and k-tile
@@ -163,18 +166,11 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(OpGemm p, int tiles_n) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) acc[h][i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int KT = (p.K + kTK - 1) / kTK;
-    if (KT > 0) {
-        load(0);
-        store(lds[0]);
-        __syncthreads();
-    }
-    for (int kt = 0; kt < KT; ++kt) {
-        if (kt + 1 < KT) load((kt + 1) * kTK);
-        const float * As = lds[kt & 1];
+    // `steps` 16-deep steps of the k-tile in buf
+    auto multiply = [&](const float * As, auto steps) {
         const float * Bs = As + A_SZ;
 #pragma unroll
-        for (int s = 0; s < kTK / 16; ++s) {
+        for (int s = 0; s < decltype(steps)::value; ++s) {
             v4f a[TM], b[TN];
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -196,44 +192,76 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(OpGemm p, int tiles_n) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) acc[e % NA][i][j] = mfma_16x16x4(b[j][e], a[i][e], acc[e % NA][i][j]);
+                    for (int j = 0; j < TN; ++j) {
+                        v4f & c = acc[e % NA][i][j];
+                        c = VC ? mfma_16x16x4(b[j][e], a[i][e], c) : mfma_16x16x4(a[i][e], b[j][e], c);
+                    }
         }
-        if (kt + 1 < KT) store(lds[(kt + 1) & 1]);
+    };
+    const int KT = (p.K + kTK - 1) / kTK;
+    if (KT > 0) {
+        load(0);
+        store(lds[0]);
         __syncthreads();
+    }
+    for (int kt = 0; kt + 1 < KT; ++kt) {
+        load((kt + 1) * kTK);
+        multiply(lds[kt & 1], std::integral_constant<int, kTK / 16>{});
+        store(lds[(kt + 1) & 1]);
+        __syncthreads();
+    }
+    // the last k-tile; its upper half is skipped where it holds none of K
+    if (KT > 0) {
+        if (p.K - (KT - 1) * kTK > kTK / 2) multiply(lds[(KT - 1) & 1], std::integral_constant<int, kTK / 16>{});
+        else multiply(lds[(KT - 1) & 1], std::integral_constant<int, kTK / 32>{});
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-        const int row = m0 + wm + i * 16 + lr;
-        if (row >= p.M) continue;
-        const float rbias = p.bias && p.bias_mode == 2 ? p.bias[row] : 0.0f;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const int col = n0 + wn + j * 16 + 4 * g;
-            if (col >= p.N) continue;
             v4f v = acc[0][i][j];
             if constexpr (NA == 2) v += acc[1][i][j];
-            float * dst = C + (int64_t)row * p.ldc + col;
-            const int nc = min(4, p.N - col);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (p.bias && e < nc) v[e] = (p.bias_mode == 2 ? rbias : p.bias[col + e]) + v[e];
-            if (p.vec_c && nc == 4) {
-                if (p.accumulate) v = *reinterpret_cast<const v4f *>(dst) + v;
-                *reinterpret_cast<v4f *>(dst) = v;
-            } else {
+            if constexpr (VC) {
+                const int row = m0 + wm + i * 16 + lr, col = n0 + wn + j * 16 + 4 * g;
+                if (row >= p.M || col >= p.N) continue;
+                float * dst = C + (int64_t)row * p.ldc + col;
+                const int nc = min(4, p.N - col);
+                const float rbias = p.bias && p.bias_mode == 2 ? p.bias[row] : 0.0f;
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (e < nc) dst[e] = p.accumulate ? dst[e] + v[e] : v[e];
+                    if (p.bias && e < nc) v[e] = (p.bias_mode == 2 ? rbias : p.bias[col + e]) + v[e];
+                if (nc == 4) {
+                    if (p.accumulate) v = *reinterpret_cast<const v4f *>(dst) + v;
+                    *reinterpret_cast<v4f *>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (e < nc) dst[e] = p.accumulate ? dst[e] + v[e] : v[e];
+                }
+            } else {
+                const int row = m0 + wm + i * 16 + 4 * g, col = n0 + wn + j * 16 + lr;
+                if (col >= p.N) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (row + e >= p.M) continue;
+                    if (p.bias) v[e] = p.bias[p.bias_mode == 2 ? row + e : col] + v[e];
+                    float * dst = C + (int64_t)(row + e) * p.ldc + col;
+                    *dst = p.accumulate ? *dst + v[e] : v[e];
+                }
             }
         }
     }
 }
 
 template <int BM, int BN>
-void launch_gemm_f32(const OpGemm & p, bool bt, bool va, bool vb, unsigned batch, hipStream_t s) {
+void launch_gemm_f32(const OpGemm & p, bool bt, bool va, bool vb, bool vc, unsigned batch, hipStream_t s) {
     const int tn = (p.N + BN - 1) / BN;
     const dim3 grid((unsigned)(((p.M + BM - 1) / BM) * tn), 1, batch), blk(256);
-#define SANA_GEMM32(T, A, B) hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, T, A, B>), grid, blk, 0, s, p, tn)
+#define SANA_GEMM32(T, A, B)                                                                                  \
+    do {                                                                                                      \
+        if (vc) hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, T, A, B, true>), grid, blk, 0, s, p, tn);         \
+        else hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, T, A, B, false>), grid, blk, 0, s, p, tn);           \
+    } while (0)
     if (bt) {
         if (va && vb) SANA_GEMM32(true, 4, 4);
         else if (va) SANA_GEMM32(true, 4, 1);
@@ -703,17 +731,20 @@ int sana_op_gemm_f32(const float * A, int64_t lda, int64_t strideA, const float 
     if (bias && bias_mode != 1 && bias_mode != 2) return fail("bias_mode must be 1 (per column) or 2 (per row)");
     if ((M + 63) / 64 > 65535) return fail("gemm M too large");
     OpGemm p{A, B, bias, C, lda, ldb, ldc, strideA, strideB, strideC, (int)M, (int)N, (int)K, bias_mode,
-             accumulate ? 1 : 0, 0};
+             accumulate ? 1 : 0};
     // 16-byte accesses: base, row stride, batch stride and the contiguous extent all multiples of 4 elements
     const bool va = aligned16(A) && lda % 4 == 0 && K % 4 == 0 && (batch == 1 || strideA % 4 == 0);
     const bool vb = aligned16(B) && ldb % 4 == 0 && (b_transposed ? K : N) % 4 == 0 && (batch == 1 || strideB % 4 == 0);
-    p.vec_c = aligned16(C) && ldc % 4 == 0 && (batch == 1 || strideC % 4 == 0);
+    const bool vc = aligned16(C) && ldc % 4 == 0 && (batch == 1 || strideC % 4 == 0);
     // The tile with the least modelled time: `fixed` + `round` per round of 256
     // workgroups, both measured at K = 1152 (us x 10; 64 to 16384 rows, 1152
     // columns, within 10 %).  Small tiles have the shorter k-step chain, large
     // ones fewer LDS reads per product.  2048 x 1152: 32x32 72 us, 64x32 65, 64x96
     // 73; 512 rows 27, 31, 44; 4096 rows 129, 111, 103; 64 products of 4096 x 72
-    // x 300: 203, 181, 164 (64x64 and 32x64 lie within 1 % of these three).
+    // x 300: 203, 181, 164 (64x64 and 32x64 lie within 1 % of these three).  B [K, N]
+    // that is read float by float over few k-tiles waits for its loads: there
+    // the middle tile, with twice the workgroups per CU, instead of the largest
+    // (16 products of 1023 x 1021 x 40: 39.6 -> 35.7 us).
     struct {
         int64_t m, n, round, fixed;
     } const tiles[3] = {{64, 96, 304, 125}, {64, 32, 110, 105}, {32, 32, 70, 90}};
@@ -722,6 +753,7 @@ int sana_op_gemm_f32(const float * A, int64_t lda, int64_t strideA, const float 
     for (int i = 0; i < 3; ++i) {
         const int64_t t = ((M + tiles[i].m - 1) / tiles[i].m) * ((N + tiles[i].n - 1) / tiles[i].n) * batch;
         const int64_t cost = tiles[i].fixed + (t + 255) / 256 * tiles[i].round;
+        if (i == 0 && !b_transposed && !vb && K <= 96) continue;
         if (t / batch < (1 << 24) && cost < best_cost) {  // a launch holds fewer than 2^32 threads per axis
             best = i;
             best_cost = cost;
@@ -729,9 +761,9 @@ int sana_op_gemm_f32(const float * A, int64_t lda, int64_t strideA, const float 
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bt = b_transposed != 0;
-    if (best == 0) launch_gemm_f32<64, 96>(p, bt, va, vb, (unsigned)batch, s);
-    else if (best == 1) launch_gemm_f32<64, 32>(p, bt, va, vb, (unsigned)batch, s);
-    else launch_gemm_f32<32, 32>(p, bt, va, vb, (unsigned)batch, s);
+    if (best == 0) launch_gemm_f32<64, 96>(p, bt, va, vb, vc, (unsigned)batch, s);
+    else if (best == 1) launch_gemm_f32<64, 32>(p, bt, va, vb, vc, (unsigned)batch, s);
+    else launch_gemm_f32<32, 32>(p, bt, va, vb, vc, (unsigned)batch, s);
     return launched("gemm_f32");
 }
 
