@@ -83,6 +83,7 @@ def test_gemm_f32_nonfinite(L):
 
 @pytest.mark.parametrize("BH,Nq,Nk,D", [(1, 1, 1, 4), (3, 17, 15, 16), (2, 100, 0, 32), (72, 1024, 1024, 32),
                                         (5, 33, 1000, 32), (2, 4096, 777, 72), (32, 529, 529, 72), (2, 40, 300, 80),
+                                        (36, 4, 4, 32), (2, 5, 4, 72), (3, 4, 5, 32),
                                         (3, 64, 64, 48), (2, 50, 60, 84), (2, 50, 60, 30), (1, 300, 4096, 64)])
 @pytest.mark.parametrize("alias", [False, True])
 def test_linear_attention_f32(L, BH, Nq, Nk, D, alias):
