@@ -1114,11 +1114,17 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     //    5760 x 1152 135 -> 129; 8192^3 945 -> 1105 TFLOP/s).  Their waves read
     //    half of the LDS bytes per product of 64 x 64 ones;
     //  * otherwise 128x128 tiles with two stages, two workgroups per CU.
-    //  The last four use schedule 2 (against 1, 16384 rows: 128x192 stores and
-    //  q|k|v 260 -> 256 and 163 -> 156 us, K = 2880 residuals 138 -> 136.5; 128x128
-    //  q|k|v of two 2048-row launches 45.2 -> 43.0), except that the 128x192
-    //  residual GEMMs with K <= 1152 keep 8 waves (4 x 2) and schedule 1 (72 us
-    //  against 74).
+    //  These use schedule 2 (against 1, 16384 rows: 128x192 stores and q|k|v 260 ->
+    //  256 and 163 -> 156 us, K = 2880 residuals 138 -> 136.5; 128x128 q|k|v of two
+    //  2048-row launches 45.2 -> 43.0), except
+    //  - the at most 5 row tiles above;
+    //  - 128x192 residual GEMMs with K <= 1152: 8 waves (4 x 2) and schedule 1 (72 us
+    //    against 74);
+    //  - two rounds of 128x128 q|k|v of which the second is less than half full, the
+    //    same 8 waves and schedule 1, and 128x192 beside another launch with 1.5 to
+    //    1.6 rounds, schedule 1 (steps of 36 x 36 and 40 x 40 tokens 7.23 -> 7.13 and
+    //    7.70 -> 7.37 ms; from 14 row panels on, 41 x 41 tokens, schedule 2 is the
+    //    faster one again).
     // (tile counts are scaled by the launches that share the CUs, p.co, and
     // by the products of a batched launch)
     // Grids of few tiles leave most CUs idle and each workgroup with a chain of
@@ -1181,8 +1187,10 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
         return launch<128, 128, 4, 2, 2, 1>(p, s);
     if (t192 >= kSlots * 3 / 2 || one_round192) {
         if (p.mode == kGemmResidual && p.K <= 1152) return launch<128, 192, 4, 2, 2, 1>(p, s);
+        if (co > 1 && t192 >= kSlots * 3 / 2 && t192 < kSlots * 8 / 5) return launch<128, 192, 2, 2, 2, 1>(p, s);
         return launch<128, 192, 2, 2, 2, 2>(p, s);
     }
+    if (p.mode == kGemmQKV && t128 > kSlots && t128 < kSlots * 3 / 2) return launch<128, 128, 4, 2, 2, 1>(p, s);
     return launch<128, 128, 2, 2, 2, 2>(p, s);
 }
 
