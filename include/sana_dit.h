@@ -215,8 +215,7 @@ int sana_dit_time_embed(sana_dit * ctx, const float * t, int64_t B, float * embe
 /* Measurement hook (no counterpart in the reference): average duration (ms)
  * over `iters` back-to-back eager launches of one kernel of the blocks, launched
  * exactly as the last forward launched it -- the same kernel instantiation and
- * shape (one batch row of a CFG pair per launch when the forward ran the pair as
- * two chains), on the forward's own buffers, which it overwrites.  Launch i
+ * shape (half the batch per launch when the forward ran it as two chains), on the forward's own buffers, which it overwrites.  Launch i
  * uses block i mod layers, so weights stream from HBM as in the forward.
  * which: 0 QKV GEMM, 1 attn-out GEMM (+ gated residual), 2 cross-q GEMM,
  * 3 cross-out GEMM (+ residual), 4 FFN inverted GEMM (+ SiLU), 5 FFN point GEMM

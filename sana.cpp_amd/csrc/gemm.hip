@@ -1111,7 +1111,7 @@ hipError_t gemm(const GemmParams & p_in, hipStream_t s) {
     //    tiles where their rounds of 256 workgroups, 1.82 of a round of 512 of
     //    128x128 each (128x192: 1.41), come to less (us, before -> after: 738 x
     //    18432 x 2304 gate | up 90 -> 75; 4096 x 3456 x 1152 48.4 -> 42.5; 8192 x
-    //    5760 x 1152 135 -> 129; 8192^3 945 -> 1105 TFLOP/s).  Their waves read
+    //    5760 x 1152 with SiLU 146 -> 140; 8192^3 945 -> 1105 TFLOP/s).  Their waves read
     //    half of the LDS bytes per product of 64 x 64 ones;
     //  * otherwise 128x128 tiles with two stages, two workgroups per CU.
     //  These use schedule 2 (against 1, 16384 rows: 128x192 stores and q|k|v 260 ->

@@ -839,8 +839,9 @@ void attention_by_products(sana_gemma * g, const std::vector<Seq> & seqs, int wi
 
 // decode_embeddings (src/gemma_encoder.cpp:95-152) on device token ids, for
 // one or more independent sequences at once: their rows share every
-// per-token kernel (norms, the projections, GeGLU) and only the attention
-// (RoPE positions, scores, softmax, P.V) runs per sequence.  Each row's
+// per-token kernel (norms, the projections, GeGLU), and RoPE and the one-pass
+// attention take all sequences in one launch each, positions and keys kept to
+// a row's own sequence (attention_by_products runs per sequence).  Each row's
 // result is bit-identical to encoding its sequence alone: the per-row
 // arithmetic and its order do not depend on the other rows.
 void encode(sana_gemma * g, const std::vector<Seq> & seqs, hipStream_t s) {

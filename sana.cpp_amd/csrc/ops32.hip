@@ -61,10 +61,10 @@ constexpr int kTK = 32;
 // covers 16 consecutive columns of four rows (16 products of 1023 x 1021 x 64 50.2 ->
 // 34.8 us; as single elements of the transposed tile those were 16 bytes apart).
 //
-// Measured on MI355X: 2048 x 1152 x 1152 65 us (84 TFLOP/s); with the other
+// Measured on MI355X: 2048 x 1152 x 1152 60 us (90 TFLOP/s); with the other
 // kernels of this file the fp32 self-attention block (2 x 1024 tokens, four
-// such products) went from 1316 to 288 us and the cross-attention block (2 x
-// 256 tokens, 300 keys) from 787 to 139 us, against a 64 x 64 tile with
+// such products) went from 1318 to 283 us and the cross-attention block (2 x
+// 256 tokens, 300 keys) from 785 to 138 us, against a 64 x 64 tile with
 // single-buffered 16-deep k-tiles and two barriers each.
 template <int BM, int BN, bool BT, int VA, int VB, bool VC>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(OpGemm p, int tiles_n) {

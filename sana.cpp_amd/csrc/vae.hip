@@ -217,8 +217,9 @@ __global__ __launch_bounds__(256) void vae_dw5x5_kernel(const f16 * __restrict__
     for (int k = 0; k < XS; ++k)
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[k][e] = 0.0f;
+    constexpr int kRows = XS == 1 ? 5 : 1;
     auto taps = [&](auto edge) {
-#pragma unroll (XS == 1 ? 5 : 1)
+#pragma unroll kRows
         for (int ky = 0; ky < 5; ++ky) {
             const int dy = ky - 2;
             const bool row_in = !edge || (yy + dy >= 0 && yy + dy < H);

@@ -108,9 +108,9 @@ def test_forward_4096px_vs_reference(full_model):
 
 @pytest.mark.parametrize("masked", [False, True], ids=["nomask", "mask"])
 def test_step_device_matches_context_then_forward(full_model, masked):
-    """sana_dit_step_device (caption projection, cross K/V and forward in one
-    graph, the forward's head beside the context GEMMs) gives the noise
-    prediction of sana_dit_set_context + sana_dit_forward bit for bit."""
+    """sana_dit_step_device (caption projection, cross K/V and forward in one call,
+    the forward's head beside the context GEMMs) gives the noise prediction of
+    sana_dit_set_context + sana_dit_forward bit for bit."""
     import torch
     m, d = full_model
     latent = O.randn((1, 32, 32, 32), 42)
@@ -123,7 +123,7 @@ def test_step_device_matches_context_then_forward(full_model, masked):
     d_lat = torch.from_numpy(latent).to(dev)
     d_bias = torch.from_numpy(np.ascontiguousarray(bias, np.float32)).to(dev) if masked else None
     out = torch.empty((2, 32, 32, 32), device=dev)
-    for _ in range(2):  # the second call replays the captured graph
+    for _ in range(2):  # the second call replays the cached block chains
         out.fill_(float("nan"))
         d.step_device(d_cap, 300, d_bias, d_lat, (1, 32, 32, 32), 999.0, out)
         torch.cuda.synchronize()
@@ -276,8 +276,8 @@ def test_small_forward_masked_vs_oracle(small_model):
 
 
 def test_small_forward_batch2_vs_oracle(small_model):
-    """A latent batch of 2 (context batch 4): the single-chain forward, patch
-    embed reading latent row b % 2, uncond rows first."""
+    """A latent batch of 2 (context batch 4): two chains of two rows, patch embed
+    reading latent row b % 2, uncond rows first."""
     m, d = small_model
     latent = O.randn((2, 8, 8, 8), 11)
     caption = O.randn((4, 16, 96), 12)
@@ -391,9 +391,9 @@ def test_small_forward_one_chain_no_graph_vs_oracle(monkeypatch):
 
 
 def test_small_loop_graph_replays_match_direct_launches(small_model, monkeypatch):
-    """The denoise loop as one cached graph: replayed with a forward and a loop
-    of another schedule between the replays, every result equals the loop
-    launched kernel by kernel (SANA_DIT_NO_GRAPH=1, read at context creation)."""
+    """The denoise loop on the cached block chains: repeated with a forward and a
+    loop of another schedule in between, every result equals the loop launched
+    kernel by kernel (SANA_DIT_NO_GRAPH=1, read at context creation)."""
     import sana_dit
     m, d = small_model
     latent = O.randn((1, 8, 8, 8), 21)
