@@ -62,7 +62,7 @@ def test_encode_vs_oracle(name, T):
 
 
 @pytest.mark.parametrize("name,Ta,Tb", [("gqa_window", 37, 64), ("gqa_window", 20, 20), ("mqa_softcap", 5, 19),
-                                         ("gemma2_2b_2layers", 438, 300)])
+                                         ("gemma2_2b_2layers", 438, 300), ("gemma2_2b_2layers", 150, 100)])
 def test_encode_pair_equals_two_encodes(name, Ta, Tb):
     """Both sequences in one pass share the per-token kernels; every row must
     equal the separate encode of its own sequence bit for bit (attention stays
