@@ -61,10 +61,10 @@ constexpr int kTK = 32;
 // covers 16 consecutive columns of four rows (16 products of 1023 x 1021 x 64 50.2 ->
 // 34.8 us; as single elements of the transposed tile those were 16 bytes apart).
 //
-// Measured on MI355X: 2048 x 1152 x 1152 60 us (90 TFLOP/s); with the other
+// Measured on MI355X: 2048 x 1152 x 1152 59 us (92 TFLOP/s); with the other
 // kernels of this file the fp32 self-attention block (2 x 1024 tokens, four
-// such products) went from 1318 to 283 us and the cross-attention block (2 x
-// 256 tokens, 300 keys) from 785 to 138 us, against a 64 x 64 tile with
+// such products) went from 1326 to 284 us and the cross-attention block (2 x
+// 256 tokens, 300 keys) from 785 to 136 us, against a 64 x 64 tile with
 // single-buffered 16-deep k-tiles and two barriers each.
 template <int BM, int BN, bool BT, int VA, int VB, bool VC>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(OpGemm p, int tiles_n) {
@@ -206,6 +206,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(OpGemm p, int tiles_n) {
     }
     for (int kt = 0; kt + 1 < KT; ++kt) {
         load((kt + 1) * kTK);
+        __builtin_amdgcn_sched_barrier(0);  // (sunk between the MFMAs, the loads come up to 5 % later)
         multiply(lds[kt & 1], std::integral_constant<int, kTK / 16>{});
         store(lds[(kt + 1) & 1]);
         __syncthreads();
@@ -737,17 +738,16 @@ int sana_op_gemm_f32(const float * A, int64_t lda, int64_t strideA, const float 
     const bool vb = aligned16(B) && ldb % 4 == 0 && (b_transposed ? K : N) % 4 == 0 && (batch == 1 || strideB % 4 == 0);
     const bool vc = aligned16(C) && ldc % 4 == 0 && (batch == 1 || strideC % 4 == 0);
     // The tile with the least modelled time: `fixed` + `round` per round of 256
-    // workgroups, both measured at K = 1152 (us x 10; 64 to 16384 rows, 1152
-    // columns, within 10 %).  Small tiles have the shorter k-step chain, large
-    // ones fewer LDS reads per product.  2048 x 1152: 32x32 72 us, 64x32 65, 64x96
-    // 73; 512 rows 27, 31, 44; 4096 rows 129, 111, 103; 64 products of 4096 x 72
-    // x 300: 203, 181, 164 (64x64 and 32x64 lie within 1 % of these three).  B [K, N]
-    // that is read float by float over few k-tiles waits for its loads: there
-    // the middle tile, with twice the workgroups per CU, instead of the largest
-    // (16 products of 1023 x 1021 x 40: 39.6 -> 35.7 us).
+    // workgroups, both measured at K = 1152 (us x 10; 64 to 4096 rows, 1152
+    // columns, within 7 %).  Small tiles have the shorter k-step chain, large
+    // ones fewer LDS reads per product.  32x32, 64x32 and 64x96, us: 400 rows 21.9,
+    // 23.6, 42.1; 1024 rows 36.6, 39.6, 42.3; 2048 61.1, 60.2, 68.3; 4096 112, 102,
+    // 96.6.  B [K, N] that is read float by float over few k-tiles waits for its
+    // loads: there the middle tile, with twice the workgroups per CU, instead of
+    // the largest (16 products of 1023 x 1021 x 40: 39.6 -> 35.7 us).
     struct {
         int64_t m, n, round, fixed;
-    } const tiles[3] = {{64, 96, 304, 125}, {64, 32, 110, 105}, {32, 32, 70, 90}};
+    } const tiles[3] = {{64, 96, 266, 156}, {64, 32, 101, 115}, {32, 32, 59, 92}};
     int best = 0;
     int64_t best_cost = INT64_MAX;
     for (int i = 0; i < 3; ++i) {

@@ -38,7 +38,8 @@ GEMMS = [
     (33, 129, 31, 1, 0, 0, 3, 0, 0), (2048, 1152, 1152, 1, 0, 0, 0, 1, 0), (600, 1152, 64, 1, 1, 0, 0, 1, 0),
     (1000, 64, 33, 7, 0, 3, 2, 2, 1), (5, 4, 0, 1, 0, 4, 0, 1, 0),
     (65, 63, 49, 1, 0, 0, 0, 2, 0), (70, 67, 16, 2, 0, 0, 1, 1, 1), (200, 101, 17, 2, 1, 1, 0, 2, 1),
-    (131, 97, 48, 1, 1, 0, 0, 0, 1), (4100, 1151, 300, 1, 0, 1, 0, 1, 1), (4100, 1151, 80, 1, 0, 0, 0, 2, 0),
+    (131, 97, 48, 1, 1, 0, 0, 0, 1), (4090, 1151, 300, 1, 0, 1, 0, 1, 1), (4090, 1151, 80, 1, 0, 0, 0, 2, 0),
+    (4090, 1152, 40, 1, 0, 0, 0, 1, 0), (4090, 1150, 44, 1, 1, 0, 1, 2, 1), (4090, 1152, 48, 1, 1, 0, 0, 2, 1),
     (1030, 1152, 40, 1, 0, 0, 0, 1, 0), (1030, 1150, 44, 1, 1, 0, 1, 2, 1), (1031, 1154, 33, 1, 0, 2, 0, 1, 0),
 ]
 
